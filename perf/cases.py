@@ -26,7 +26,6 @@ from qsrt_amd.sqg_e4m3 import sqg_xor_cheb_t12_bytes
 
 DEV = "cuda:0"
 RHO = 0.85  # correlation of neighbouring calibration channels
-LAYER_EXPERT = (7168, 2048)
 
 
 def listed():
