@@ -423,7 +423,7 @@ __device__ int boundary_argmin(const float* cost, float* red_v, int* red_i, int 
         for (int w = 1; w < kWaves; ++w)
             if (red_v[w] < bv || (red_v[w] == bv && red_i[w] < bi)) { bv = red_v[w]; bi = red_i[w]; }
     }
-    return bi;
+    return bi & (G::S - 1);  // no state compares when every cost is NaN: still a state
 }
 
 // Traceback on wave 0 alone, for tracebacks with no pass to hide behind.
