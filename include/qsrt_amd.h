@@ -27,9 +27,12 @@ int qsrt_abi_version(void);
 const char *qsrt_last_error(void);
 
 /*
- * Bytes of traceback workspace qsrt_viterbi_tiles needs for `n_tiles` tiles
- * at rate K on the current device (one 256-row decision buffer per
- * workgroup, at most one workgroup per compute unit).  0 on error.
+ * Bytes of traceback workspace qsrt_viterbi_tiles uses for `n_tiles` tiles
+ * at rate K on the current device (per workgroup, at most one per compute
+ * unit, two passes of cost checkpoints at K2..K4, two 256-row decision
+ * buffers at the other rates).  0 on error.  K2..K4 also run in two decision
+ * buffers per workgroup (2 MiB; 1 MiB at K4) on the slower recorded
+ * traceback, with the same results.
  * Replaces the workspace sizing of qsrt/sqg_quantizer.py:410-427
  * (_sqg_temp_buffers).
  */
