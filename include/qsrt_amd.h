@@ -233,6 +233,22 @@ int qsrt_decode_noalloc(const qsrt_decode_job *jobs, int n_jobs, int K, const ui
                         int out_dtype, void *stream);
 
 /*
+ * One uniform-rate matrix with the payload's own FP16 scales:
+ *   words i16 [rows / 16, cols / 16, 16 K], suh f16 [rows], svh f16 [cols]
+ *   -> out[r * out_ld + c] (bf16 or f32 as out_dtype says).
+ * The result of qsrt_decode on the FP8 matrix-core path (a LUT with
+ * |label| <= 6) with row_scale = suh / 128 and col_scale = svh, in one launch:
+ * the job rides in the kernel's arguments and the scales are widened where
+ * they are read, so nothing is uploaded or converted first and no workspace is
+ * needed.  rows and cols multiples of 128, K 2..4, words, out and lut_e4m3
+ * 16-byte aligned, out_ld >= cols and a multiple of 8.  Replaces
+ * decode_exl3_weight (qsrt/exl3_reference.py:280-302).
+ */
+int qsrt_decode_matrix_f16(const int16_t *words, int64_t rows, int64_t cols, int K, const uint16_t *suh,
+                           const uint16_t *svh, const uint8_t *lut_e4m3, int out_dtype, void *out, int64_t out_ld,
+                           void *stream);
+
+/*
  * C[M, N] += alpha * A^T (B - B2) on the matrix cores, all row-major:
  *   A [K, M] (lda), B and B2 [K, N] (ldb), C [M, N] f32 (ldc).
  *   dtype 0: f32 operands (16-byte aligned, lda/ldb multiples of 4), exact

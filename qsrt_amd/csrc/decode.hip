@@ -105,23 +105,26 @@ __device__ __forceinline__ void cursor_next(const Job* jobs, Cursor& cu) {
     }
 }
 
-struct BlockCtx {
+template <typename Scale>
+struct BlockCtxOf {
     const int16_t* words;  // tile (8 br, 8 bc) of the block
     int64_t trs, tcs;
-    const float* su;       // row 128 br
-    const float* sv;       // col 128 bc
+    const Scale* su;       // row 128 br
+    const Scale* sv;       // col 128 bc
     char* out;             // element (128 br, 128 bc)
     int64_t ld;
 };
+using BlockCtx = BlockCtxOf<float>;
 
-__device__ __forceinline__ BlockCtx block_ctx(const Job* jobs, const Cursor& cu, int out_size) {
+template <typename Scale = float>
+__device__ __forceinline__ BlockCtxOf<Scale> block_ctx(const Job* jobs, const Cursor& cu, int out_size) {
     const Job& J = jobs[cu.j];
-    BlockCtx x;
+    BlockCtxOf<Scale> x;
     x.words = J.words + cu.br * J.block_row_stride + cu.bc * J.block_col_stride;
     x.trs = J.tile_row_stride;
     x.tcs = J.tile_col_stride;
-    x.su = J.row_scale + 128 * cu.br;
-    x.sv = J.col_scale + 128 * cu.bc;
+    x.su = reinterpret_cast<const Scale*>(J.row_scale) + 128 * cu.br;
+    x.sv = reinterpret_cast<const Scale*>(J.col_scale) + 128 * cu.bc;
     x.out = static_cast<char*>(J.out) + (128 * cu.br * J.out_ld + 128 * cu.bc) * out_size;
     x.ld = J.out_ld;
     return x;
@@ -129,8 +132,8 @@ __device__ __forceinline__ BlockCtx block_ctx(const Job* jobs, const Cursor& cu,
 
 // 16 bytes of the wave's tile-column: lane l < 16 K loads chunk l % (2 K) of
 // tile-row l / (2 K) (each tile is 32 K bytes of words).
-template <int K>
-__device__ __forceinline__ u32x4 fetch_words(const BlockCtx& x, int w, int lane) {
+template <int K, typename Scale>
+__device__ __forceinline__ u32x4 fetch_words(const BlockCtxOf<Scale>& x, int w, int lane) {
     if (lane >= 16 * K) return u32x4{0u, 0u, 0u, 0u};
     const int a = lane / (2 * K), q = lane % (2 * K);
     const int16_t* tile = x.words + a * x.trs + w * x.tcs;
@@ -336,7 +339,7 @@ void decode_fp32_kernel(const Job* __restrict__ jobs, int n_jobs, int64_t total_
 // label exchange and no barrier after the LUT load, so the workgroup's twelve
 // waves drift into different phases (gathers, MFMAs, VALU, stores) and keep
 // every pipe busy at once.
-constexpr int kBlockWaves = 12;  // one workgroup of 12 waves per CU (3 per SIMD)
+constexpr int kBlockWaves = 12;  // one workgroup of at most 12 waves per CU (3 per SIMD)
 constexpr int kBlockThreads = 64 * kBlockWaves;
 constexpr int kSliceBytes = 2048;  // half an output tile-row of bf16 (16 rows x 128 B); a tile-column's words
 constexpr int kScaleBytes = 1024;  // a block's su (128 f32) and fp16-paired sv (128 x 2 fp16)
@@ -354,7 +357,8 @@ template <typename T>
 __device__ __forceinline__ T* sgpr_ptr(T* p) {
     return reinterpret_cast<T*>(sgpr64(reinterpret_cast<int64_t>(p)));
 }
-__device__ __forceinline__ BlockCtx uniform_ctx(BlockCtx x) {
+template <typename Scale>
+__device__ __forceinline__ BlockCtxOf<Scale> uniform_ctx(BlockCtxOf<Scale> x) {
     x.words = sgpr_ptr(x.words);
     x.trs = sgpr64(x.trs);
     x.tcs = sgpr64(x.tcs);
@@ -365,28 +369,68 @@ __device__ __forceinline__ BlockCtx uniform_ctx(BlockCtx x) {
     return x;
 }
 
-template <int K, typename OutT>
+// Where a launch's jobs are: a table in device memory with FP32 scales (row
+// scales already divided by 128), or one job in the kernel's own argument with
+// the payload's FP16 scales, which needs no upload and no conversion launch.
+struct JobTable {
+    typedef float Scale;
+    const Job* table;
+    __device__ const Job* jobs() const { return table; }
+    __device__ static float row_scale(float v) { return v; }
+};
+struct OneJob {
+    typedef _Float16 Scale;
+    Job job;
+    __device__ const Job* jobs() const { return &job; }
+    __device__ static float row_scale(_Float16 v) { return static_cast<float>(v) * 0.0078125f; }
+};
+
+template <int K, typename OutT, typename Source>
 __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(3, 3)))
-void decode_block_wave_kernel(const Job* __restrict__ jobs, int n_jobs, int64_t total_blocks,
+void decode_block_wave_kernel(const Source source, int n_jobs, int64_t total_blocks,
                               const uint8_t* __restrict__ lut) {
     static_assert(sizeof(OutT) == 2 || sizeof(OutT) == 4, "bf16 or f32 output");
+    typedef typename Source::Scale Scale;
+    typedef const __attribute__((address_space(1))) Scale* gscale;
     __shared__ __attribute__((aligned(16))) uint8_t lut_s[65536];
     __shared__ __attribute__((aligned(16))) uint8_t slices[kBlockWaves * kSliceBytes];
     __shared__ __attribute__((aligned(16))) uint8_t scales[kBlockWaves * kScaleBytes];
 
-    for (int i = threadIdx.x; i < 65536 / 16; i += kBlockThreads)
-        reinterpret_cast<uint4*>(lut_s)[i] = reinterpret_cast<const uint4*>(lut)[i];
-    __syncthreads();  // the kernel's only barrier
-
+    const Job* const jobs = source.jobs();
+    const int waves = static_cast<int>(blockDim.x) >> 6;
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int64_t gw = static_cast<int64_t>(blockIdx.x) * kBlockWaves + w;
-    const int64_t nw = static_cast<int64_t>(gridDim.x) * kBlockWaves;
+    const int64_t gw = static_cast<int64_t>(blockIdx.x) * waves + w;
+    const int64_t nw = static_cast<int64_t>(gridDim.x) * waves;
     const int64_t begin = sgpr64(total_blocks * gw / nw);
     const int64_t end = sgpr64(total_blocks * (gw + 1) / nw);
+
+    // The first block's words and scales are requested ahead of the table: a wave of a small launch decodes one block.
+    const int c = lane & 15;
+    Cursor cu{};
+    BlockCtxOf<Scale> ctx{};
+    u32x4 words[8];
+    float su_n[8], sv_n[8];
+    if (begin < end) {
+        cu = cursor_at(jobs, n_jobs, begin);
+        ctx = uniform_ctx(block_ctx<Scale>(jobs, cu, sizeof(OutT)));
+#pragma unroll
+        for (int col = 0; col < 8; ++col) words[col] = fetch_words<K>(ctx, col, lane);
+#pragma unroll
+        for (int a = 0; a < 8; ++a) {
+            su_n[a] = Source::row_scale(((gscale)ctx.su)[16 * a + c]);
+            sv_n[a] = static_cast<float>(((gscale)ctx.sv)[16 * a + c]);
+        }
+    }
+    // The table goes to LDS without passing through registers, every load in flight at once: copied 16 bytes per
+    // thread and round trip, a workgroup of 4 waves spent 16 round trips on it, half of a one-block launch.
+    for (int i = w; i < 65536 / 1024; i += waves)
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(lut + 1024 * i + 16 * lane),
+                                         (__attribute__((address_space(3))) void*)(lut_s + 1024 * i), 16, 0, 0);
+    __builtin_amdgcn_s_waitcnt(0);  // vmcnt(0): the builtin's writes to LDS are not ordered by the barrier alone
+    __syncthreads();  // the kernel's only barrier
     if (begin >= end) return;
 
-    const int c = lane & 15;
     const int g = lane >> 4;
     const int rho[4] = {2 * g, 2 * g + 1, 2 * g + 8, 2 * g + 9};
     // B of tile-row 0: byte i of every register is H16[rho(i)][c] in E4M3 (+1 0x38, -1 0xB8)
@@ -414,20 +458,8 @@ void decode_block_wave_kernel(const Job* __restrict__ jobs, int n_jobs, int64_t 
 
     // Loads of a block are issued before the previous block's stores: vector-memory counters retire in issue
     // order, so a load issued after stores returns only once they have drained.
-    Cursor cu = cursor_at(jobs, n_jobs, begin);
-    BlockCtx ctx = uniform_ctx(block_ctx(jobs, cu, sizeof(OutT)));
-    u32x4 words[8];
-#pragma unroll
-    for (int col = 0; col < 8; ++col) words[col] = fetch_words<K>(ctx, col, lane);
-    float su_n[8], sv_n[8];
-#pragma unroll
-    for (int a = 0; a < 8; ++a) {
-        su_n[a] = ((gf32)ctx.su)[16 * a + c];
-        sv_n[a] = ((gf32)ctx.sv)[16 * a + c];
-    }
-
     for (int64_t blk = begin; blk < end; ++blk) {
-        const BlockCtx cur = ctx;
+        const BlockCtxOf<Scale> cur = ctx;
         // ---- labels of all 64 tiles, tile-column by tile-column (high issue priority: the gathers are the
         // phase other waves' MFMA and store phases can hide behind)
         __builtin_amdgcn_s_setprio(2);
@@ -467,11 +499,11 @@ void decode_block_wave_kernel(const Job* __restrict__ jobs, int n_jobs, int64_t 
         for (int a = 0; a < 8; ++a) su_n[a] = sv_n[a] = 0.f;  // likewise
         if (more) {
             cursor_next(jobs, cu);
-            ctx = uniform_ctx(block_ctx(jobs, cu, sizeof(OutT)));
+            ctx = uniform_ctx(block_ctx<Scale>(jobs, cu, sizeof(OutT)));
 #pragma unroll
             for (int a = 0; a < 8; ++a) {
-                su_n[a] = ((gf32)ctx.su)[16 * a + c];
-                sv_n[a] = ((gf32)ctx.sv)[16 * a + c];
+                su_n[a] = Source::row_scale(((gscale)ctx.su)[16 * a + c]);
+                sv_n[a] = static_cast<float>(((gscale)ctx.sv)[16 * a + c]);
             }
         }
         // ---- output tile-rows in Gray-code order; the left MFMAs at priority 1, the rest at 0
@@ -584,25 +616,34 @@ void decode_block_wave_kernel(const Job* __restrict__ jobs, int n_jobs, int64_t 
     }
 }
 
-// One workgroup of kBlockWaves waves per CU (fewer when there are fewer blocks).
-template <int K>
-void launch_block_wave_k(const Job* jobs, int n_jobs, int64_t total, const uint8_t* lut, int out_dtype, int cus,
+// One workgroup per CU.  Its waves are as many as share the blocks out evenly
+// over the rounds that twelve waves per CU would take: 896 blocks (one
+// 7168 x 2048 matrix) run as 224 workgroups of 4 waves, not as 75 of 12 with
+// the other CUs idle (32.5 -> 18.9 us at K3 under the trace, the table copy
+// included).  Cutting such blocks further, into parts of their tile-rows on
+// twice the waves, was no faster (20.3 us): the label phase, which every part
+// repeats, is what a lone wave takes its time for.
+template <int K, typename Source>
+void launch_block_wave_k(const Source& source, int n_jobs, int64_t total, const uint8_t* lut, int out_dtype, int cus,
                          hipStream_t stream) {
-    const int64_t groups = (total + kBlockWaves - 1) / kBlockWaves;
-    const unsigned grid = static_cast<unsigned>(std::min<int64_t>(cus, groups));
+    const int64_t per_round = static_cast<int64_t>(cus) * kBlockWaves;
+    const int64_t rounds = (total + per_round - 1) / per_round;
+    const int64_t waves = (total + rounds * cus - 1) / (rounds * cus);
+    const unsigned grid = static_cast<unsigned>(std::min<int64_t>(cus, (total + waves - 1) / waves));
+    const dim3 block(static_cast<unsigned>(64 * waves));
     if (out_dtype == 0)
-        hipLaunchKernelGGL((decode_block_wave_kernel<K, __bf16>), dim3(grid), dim3(kBlockThreads), 0, stream, jobs,
-                           n_jobs, total, lut);
+        hipLaunchKernelGGL((decode_block_wave_kernel<K, __bf16, Source>), dim3(grid), block, 0, stream, source, n_jobs,
+                           total, lut);
     else
-        hipLaunchKernelGGL((decode_block_wave_kernel<K, float>), dim3(grid), dim3(kBlockThreads), 0, stream, jobs,
-                           n_jobs, total, lut);
+        hipLaunchKernelGGL((decode_block_wave_kernel<K, float, Source>), dim3(grid), block, 0, stream, source, n_jobs,
+                           total, lut);
 }
 
 template <int K, bool FP8>
 void launch(const Job* jobs, int n_jobs, int64_t total, const uint8_t* lut, int out_dtype, int cus,
             hipStream_t stream) {
     if constexpr (FP8) {
-        launch_block_wave_k<K>(jobs, n_jobs, total, lut, out_dtype, cus, stream);
+        launch_block_wave_k<K>(JobTable{jobs}, n_jobs, total, lut, out_dtype, cus, stream);
     } else {
         const unsigned grid = static_cast<unsigned>(std::min<int64_t>(2 * static_cast<int64_t>(cus), total));  // 2 per CU
         if (out_dtype == 0)
@@ -633,13 +674,32 @@ __global__ __launch_bounds__(64) void upload_jobs_kernel(JobChunk chunk, Job* __
     if (i < chunk.count) dst[i] = chunk.jobs[i];
 }
 
-bool job_ok(const qsrt_decode_job& s) {
+bool strides_ok(const qsrt_decode_job& s) {
     return s.words && s.row_scale && s.col_scale && s.out && s.rows >= 0 && s.cols >= 0 && s.rows % 128 == 0 &&
            s.cols % 128 == 0 && s.out_ld >= s.cols && s.out_ld % 8 == 0 &&
            reinterpret_cast<uintptr_t>(s.words) % 16 == 0 && s.tile_row_stride % 8 == 0 &&
            s.tile_col_stride % 8 == 0 && s.block_row_stride % 8 == 0 && s.block_col_stride % 8 == 0 &&
-           reinterpret_cast<uintptr_t>(s.out) % 16 == 0 && reinterpret_cast<uintptr_t>(s.col_scale) % 16 == 0 &&
+           reinterpret_cast<uintptr_t>(s.out) % 16 == 0;
+}
+
+bool job_ok(const qsrt_decode_job& s) {
+    return strides_ok(s) && reinterpret_cast<uintptr_t>(s.col_scale) % 16 == 0 &&
            reinterpret_cast<uintptr_t>(s.row_scale) % 16 == 0;
+}
+
+Job device_job(const qsrt_decode_job& s, int64_t first_block) {
+    return Job{s.words,
+               s.tile_row_stride,
+               s.tile_col_stride,
+               s.block_row_stride ? s.block_row_stride : 8 * s.tile_row_stride,
+               s.block_col_stride ? s.block_col_stride : 8 * s.tile_col_stride,
+               s.row_scale,
+               s.col_scale,
+               s.out,
+               s.out_ld,
+               static_cast<int32_t>(s.rows / 128),
+               static_cast<int32_t>(s.cols / 128),
+               first_block};
 }
 
 // Most jobs the no-allocation decode holds (its job table is `scratch`).
@@ -719,18 +779,7 @@ int qsrt_decode_prepare(const qsrt_decode_job* jobs, int n_jobs, int K, void* wo
     for (int i = 0; i < n_jobs; ++i) {
         const qsrt_decode_job& s = jobs[i];
         if (s.rows == 0 || s.cols == 0) continue;
-        chunk.jobs[chunk.count++] = Job{s.words,
-                                        s.tile_row_stride,
-                                        s.tile_col_stride,
-                                        s.block_row_stride ? s.block_row_stride : 8 * s.tile_row_stride,
-                                        s.block_col_stride ? s.block_col_stride : 8 * s.tile_col_stride,
-                                        s.row_scale,
-                                        s.col_scale,
-                                        s.out,
-                                        s.out_ld,
-                                        static_cast<int32_t>(s.rows / 128),
-                                        static_cast<int32_t>(s.cols / 128),
-                                        total};
+        chunk.jobs[chunk.count++] = device_job(s, total);
         total += (s.rows / 128) * (s.cols / 128);
         if (chunk.count == kUploadChunk || i == n_jobs - 1) {
             hipLaunchKernelGGL(upload_jobs_kernel, dim3(1), dim3(64), 0, stream, chunk, table + kept);
@@ -798,4 +847,31 @@ extern "C" int qsrt_decode_noalloc(const qsrt_decode_job* jobs, int n_jobs, int 
     qsrt_decode_plan plan;
     if (const int rc = qsrt_decode_prepare(jobs, n_jobs, K, table, sizeof(Job) * kStaticJobs, &plan, stream)) return rc;
     return qsrt_decode_execute(&plan, lut_e4m3, exact_fp8, out_dtype, stream);
+}
+
+extern "C" int qsrt_decode_matrix_f16(const int16_t* words, int64_t rows, int64_t cols, int K, const uint16_t* suh,
+                                      const uint16_t* svh, const uint8_t* lut_e4m3, int out_dtype, void* out,
+                                      int64_t out_ld, void* stream_handle) {
+    if (out_dtype != 0 && out_dtype != 1) return qsrt::fail(qsrt::kBadArgument, "out_dtype must be 0 (bf16) or 1 (f32)");
+    if (K < 2 || K > 4) return qsrt::fail(qsrt::kBadArgument, "K%d decode is not supported (K2..K4)", K);
+    const qsrt_decode_job s = {words, cols * K, 16 * K, reinterpret_cast<const float*>(suh),
+                               reinterpret_cast<const float*>(svh), out, out_ld, rows, cols, 0, 0};
+    if (!strides_ok(s) || reinterpret_cast<uintptr_t>(suh) % 2 || reinterpret_cast<uintptr_t>(svh) % 2)
+        return qsrt::fail(qsrt::kBadArgument,
+                          "decode matrix: need rows, cols multiples of 128, out_ld >= cols and a multiple of 8, 16-byte "
+                          "aligned words and out, non-null pointers");
+    if (rows / 128 >= (1 << 30) || cols / 128 >= (1 << 30))
+        return qsrt::fail(qsrt::kBadArgument, "decode matrix is too large");
+    if (rows == 0 || cols == 0) return qsrt::kOk;
+    if (!lut_e4m3) return qsrt::fail(qsrt::kBadArgument, "null pointer argument");
+    if (reinterpret_cast<uintptr_t>(lut_e4m3) % 16) return qsrt::fail(qsrt::kBadArgument, "LUT must be 16-byte aligned");
+    int cus = 0;
+    if (const int rc = qsrt::current_cu_count(&cus)) return rc;
+    const OneJob source{device_job(s, 0)};
+    const int64_t total = (rows / 128) * (cols / 128);
+    auto* launch = K == 2 ? launch_block_wave_k<2, OneJob> : K == 3 ? launch_block_wave_k<3, OneJob>
+                                                                    : launch_block_wave_k<4, OneJob>;
+    launch(source, 1, total, lut_e4m3, out_dtype, cus, static_cast<hipStream_t>(stream_handle));
+    QSRT_HIP_TRY(hipGetLastError());
+    return qsrt::kOk;
 }

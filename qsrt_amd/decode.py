@@ -26,7 +26,9 @@ _OUT = {torch.bfloat16: 0, torch.float32: 1}
 def _check_lut(lut: torch.Tensor, device) -> torch.Tensor:
     if lut.dtype != torch.uint8 or lut.numel() != 1 << 16:
         raise ValueError("decode LUT must be uint8[65536] E4M3 bytes")
-    lut = _lut_on(lut.reshape(-1), torch.device(device))
+    # a flat table stays the caller's own tensor, which remembers its label bound per version (a reduction and a host
+    # synchronisation otherwise paid on every call)
+    lut = _lut_on(lut if lut.ndim == 1 else lut.reshape(-1), torch.device(device))
     if lut.data_ptr() % 16:
         lut = lut.clone()
     return lut
@@ -36,6 +38,13 @@ def _scale(v: torch.Tensor, n: int, device, divide: float = 1.0) -> torch.Tensor
     if v.ndim != 1 or v.numel() != n:
         raise ValueError(f"scale vector must contain exactly {n} values")
     return (v.to(device=device, dtype=torch.float32) / divide).contiguous()
+
+
+def _payload_scale(v: torch.Tensor, n: int, device) -> bool:
+    """Whether ``v`` is a payload's scale vector as the kernel reads it."""
+
+    return (v.dtype == torch.float16 and v.ndim == 1 and v.numel() == n and v.device == device
+            and (v.stride(0) == 1 or n == 1))
 
 
 def _run(jobs: list, bits: int, lut: torch.Tensor, out_dtype, device) -> None:
@@ -71,12 +80,22 @@ def decode_words(words: torch.Tensor, suh: torch.Tensor, svh: torch.Tensor, bits
     dev = words.device
     words = words.contiguous()
     lut = _check_lut(lut, dev)
-    su = _scale(suh, k, dev, 128.0)
-    sv = _scale(svh, n, dev)
+    direct = _payload_scale(suh, k, dev) and _payload_scale(svh, n, dev) and _lut_abs_max(lut) <= FP8_EXACT_MAX_LABEL
+    if not direct:
+        su = _scale(suh, k, dev, 128.0)
+        sv = _scale(svh, n, dev)
     if out is None:
         out = torch.empty((k, n), dtype=out_dtype, device=dev)
     elif out.shape != (k, n) or out.dtype != out_dtype or out.stride(1) != 1:
         raise ValueError("out must be a row-major [K, N] tensor of out_dtype")
+    if direct:  # the payload's own FP16 scales: one launch, nothing uploaded or converted before it
+        _native.check(
+            _native.lib().qsrt_decode_matrix_f16(words.data_ptr(), k, n, bits, suh.data_ptr(), svh.data_ptr(),
+                                                 lut.data_ptr(), _OUT[out_dtype], out.data_ptr(), out.stride(0),
+                                                 _native.stream_handle(dev)),
+            "qsrt_decode_matrix_f16",
+        )
+        return out
     job = _native.DecodeJob(words.data_ptr(), nt * 16 * bits, 16 * bits, su.data_ptr(), sv.data_ptr(),
                             out.data_ptr(), out.stride(0), k, n, 0, 0)
     _run([job], bits, lut, out_dtype, dev)

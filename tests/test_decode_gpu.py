@@ -226,3 +226,27 @@ def test_decode_of_encoded_payload_equals_encoder_reconstruction():
     from qsrt_amd.exl3_reference import decode_exl3_weight
     ref = decode_exl3_weight(Q.unpack_trellis_states(tensors["trellis"], 3), tensors["suh"], tensors["svh"], bits=3)
     assert float((got - ref).abs().max()) <= 1e-5 * float(ref.abs().max())
+
+
+@pytest.mark.parametrize("shape", ((128, 128), (128, 128 * 256), (128, 128 * 257), (24 * 128, 128 * 128), (25 * 128, 128 * 123)))
+@pytest.mark.parametrize("bits", (2, 3, 4))
+def test_payload_scales_equal_converted_scales(bits, shape):
+    """FP16 scales read by the kernel against the same values converted
+    beforehand (the job table route), at block counts around the changes of
+    waves per workgroup and of rounds: 1, 256, 257, 3072 (twelve waves on
+    every one of 256 CUs), 3075 (two rounds); a row stride wider than N."""
+
+    k, n = shape
+    print(f"[decode] K{bits} {k} x {n}, both scale routes", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(bits * 10007 + k + n)
+    words = torch.randint(-32768, 32768, (k // 16, n // 16, 16 * bits), generator=gen, device="cuda",
+                          dtype=torch.int32).to(torch.int16)
+    suh = (torch.rand(k, generator=gen, device="cuda") + 0.5).half()
+    svh = torch.randn(n, generator=gen, device="cuda").half()
+    lut = sqg_xor_cheb_t12_bytes(bits).cuda()
+    for dtype in (torch.bfloat16, torch.float32):
+        want = D.decode_words(words, suh.float(), svh.float(), bits, lut, out_dtype=dtype)
+        out = torch.zeros((k, n + 8), dtype=dtype, device="cuda")
+        got = D.decode_words(words, suh, svh, bits, lut, out_dtype=dtype, out=out[:, :n])
+        assert torch.equal(got, want)
+        assert not out[:, n:].any()
