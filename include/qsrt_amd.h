@@ -263,8 +263,8 @@ int qsrt_gemm_tn(float *C, const void *A, const void *B, const void *B2, int64_t
 
 /*
  * Device bytes qsrt_gemm_tn_ws wants as workspace for these arguments (0 when
- * the call has nothing to split: dtype 0, or a bf16 tile count that fills the
- * device's compute units in whole rounds).
+ * the call has nothing to split: an f32 product that is not A^T A, or a tile
+ * count that fills the device's compute units).
  */
 size_t qsrt_gemm_tn_workspace_bytes(const float *C, const void *A, const void *B, int64_t M, int64_t N, int64_t K,
                                     int64_t lda, int64_t ldb, int64_t ldc, int dtype);
@@ -272,10 +272,12 @@ size_t qsrt_gemm_tn_workspace_bytes(const float *C, const void *A, const void *B
 /*
  * qsrt_gemm_tn with a device workspace (16-byte aligned).  bf16: when the
  * 256 x 256 tiles do not fill the compute units in whole rounds, the tiles of
- * the last round are split along K and their partial products, written to
- * the workspace, are added to C in K order by a second kernel on the same
- * stream (the result is deterministic; it differs from the unsplit sum only
- * by FP32 rounding).  A NULL or short workspace runs every tile whole, as
+ * the last round are split along K where that is faster and their partial
+ * products, written to the workspace, are added to C in K order by a second
+ * kernel on the same stream (the result is deterministic; it differs from the
+ * unsplit sum only by FP32 rounding).  f32 with A == B and no B2 (a Gram):
+ * likewise for its 128 x 128 tiles on and above the diagonal, the only ones
+ * computed.  A NULL or short workspace runs every tile whole, as
  * qsrt_gemm_tn does.  Same operator and call sites as qsrt_gemm_tn.
  */
 int qsrt_gemm_tn_ws(float *C, const void *A, const void *B, const void *B2, int64_t M, int64_t N, int64_t K,

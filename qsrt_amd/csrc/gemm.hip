@@ -518,13 +518,174 @@ int64_t bf16_tiles(bool sym, int64_t M, int64_t N) {
     return sym ? tm * (tm + 1) / 2 : tm * tn;
 }
 
+// ---------------------------------------------------------------- FP32 Gram
+// C += alpha * X^T X with FP32 operands: only the 128 x 128 tiles on and above
+// the diagonal are computed (an off-diagonal one also adds its transpose), on
+// the MFMA loop of gemm_tn_f32_kernel.  A 2048-channel Gram has 136 such
+// tiles, half a tile per CU: K is cut into `parts` ranges, each range's
+// accumulators go to a workspace, and gram_f32_fixup adds them to C in K
+// order (deterministic).  MFMA-bound: 16384 x 2048 in all 256 tiles and one
+// workgroup per CU took 1.47 ms (0.59 of the FP32 matrix peak, half of it
+// redundant), this way 0.67 ms (0.69 of the peak, 6% redundant).
+constexpr int64_t kGramPartial = 16 * kThreads;  // f32x4 per partial tile (64 KiB)
+
+// Sum of a tile's accumulators (16-row block i of every wave's 64 x 64 block) into C and, off the diagonal, into the
+// transposed tile.  lane holds C[m0 + wm + 16 i + 4 g + r][n0 + wn + 16 j + c]
+__device__ __forceinline__ void gram_f32_epilogue(float* __restrict__ C, const f32x4 (&acc)[4], int i, int64_t M,
+                                                  int64_t ldc, float alpha, int tm, int tn, int t) {
+    const int lane = t & 63, wave = t >> 6, c = lane & 15, g = lane >> 4;
+    const int64_t row0 = static_cast<int64_t>(tm) * kBM + (wave >> 1) * 64 + 16 * i + 4 * g;
+    const int64_t col0 = static_cast<int64_t>(tn) * kBN + (wave & 1) * 64 + c;
+    if ((tm + 1) * static_cast<int64_t>(kBM) <= M && (tn + 1) * static_cast<int64_t>(kBN) <= M) {
+        float v[4][4];
+        f32x4 w[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[j][r] = C[(row0 + r) * ldc + col0 + 16 * j];
+            if (tm != tn) w[j] = *reinterpret_cast<const f32x4*>(C + (col0 + 16 * j) * ldc + row0);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) C[(row0 + r) * ldc + col0 + 16 * j] = v[j][r] + alpha * acc[j][r];
+            if (tm != tn) *reinterpret_cast<f32x4*>(C + (col0 + 16 * j) * ldc + row0) = w[j] + alpha * acc[j];
+        }
+        return;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int64_t col = col0 + 16 * j;
+        if (col >= M) continue;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            if (row0 + r >= M) continue;
+            C[(row0 + r) * ldc + col] += alpha * acc[j][r];
+            if (tm != tn) C[col * ldc + row0 + r] += alpha * acc[j][r];
+        }
+    }
+}
+
+template <bool PARTIAL>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3))) void gram_f32_kernel(
+    float* __restrict__ C, const float* __restrict__ X, int64_t M, int64_t K, int64_t ld, int64_t ldc, float alpha,
+    int tiles_m, int tiles, int parts, f32x4* __restrict__ ws) {
+    __shared__ __attribute__((aligned(16))) float As[2][kBK32][kBM + kPad32];
+    __shared__ __attribute__((aligned(16))) float Bs[2][kBK32][kBN + kPad32];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int c = lane & 15, g = lane >> 4;
+    // range-major, so the workgroups resident on an XCD walk one K range of neighbouring tiles
+    const int q = xcd_slot(static_cast<int>(blockIdx.x), tiles * parts), part = q / tiles, tile = q % tiles;
+    int tm = 0, tn = 0;
+    if (!tile_at(tile, tiles_m, tiles_m, true, tm, tn)) return;  // not reached
+    const int64_t m0 = static_cast<int64_t>(tm) * kBM, n0 = static_cast<int64_t>(tn) * kBN;
+    const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
+    const int64_t all = (K + kBK32 - 1) / kBK32;
+    const int64_t first = all * part / parts, last = all * (part + 1) / parts;
+    f32x4 acc[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    F32Chunk ch;
+    load_f32(ch, X, X, nullptr, first * kBK32, m0, n0, M, M, K, ld, ld, t);
+    store_f32(ch, As[0], Bs[0], t);
+    __syncthreads();
+    for (int64_t kc = first; kc < last; ++kc) {
+        const int cur = static_cast<int>((kc - first) & 1);
+        if (kc + 1 < last) load_f32(ch, X, X, nullptr, (kc + 1) * kBK32, m0, n0, M, M, K, ld, ld, t);
+#pragma unroll
+        for (int kk = 0; kk < kBK32 / 4; ++kk) {
+            float a[4], b[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) a[i] = As[cur][4 * kk + g][wm + 16 * i + c];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) b[j] = Bs[cur][4 * kk + g][wn + 16 * j + c];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[j], acc[i][j], 0, 0, 0);
+        }
+        if (kc + 1 < last) store_f32(ch, As[cur ^ 1], Bs[cur ^ 1], t);
+        __syncthreads();
+    }
+    if constexpr (PARTIAL) {
+        f32x4* w = ws + static_cast<int64_t>(part * tiles + tile) * kGramPartial;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) w[(4 * i + j) * kThreads + t] = acc[i][j];
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) gram_f32_epilogue(C, acc[i], i, M, ldc, alpha, tm, tn, t);
+    }
+}
+
+// Four workgroups per tile, one per 16-row block of every wave's 64 x 64 block: the ranges in K order, then C.
+__global__ __launch_bounds__(kThreads) void gram_f32_fixup(float* __restrict__ C, int64_t M, int64_t ldc, float alpha,
+                                                           int tiles_m, int tiles, int parts,
+                                                           const f32x4* __restrict__ ws) {
+    const int tile = static_cast<int>(blockIdx.x) / 4, i = static_cast<int>(blockIdx.x) % 4;
+    const int t = static_cast<int>(threadIdx.x);
+    int tm = 0, tn = 0;
+    if (!tile_at(tile, tiles_m, tiles_m, true, tm, tn)) return;  // not reached
+    const f32x4* w = ws + static_cast<int64_t>(tile) * kGramPartial + 4 * i * kThreads + t;
+    f32x4 acc[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[j] = w[j * kThreads];
+    for (int part = 1; part < parts; ++part) {
+        w += tiles * kGramPartial;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[j] += w[j * kThreads];
+    }
+    gram_f32_epilogue(C, acc, i, M, ldc, alpha, tm, tn, t);
+}
+
+// K ranges per tile.  In units of one whole tile on a CU of its own at full MFMA rate: the CU with most ranges has n of
+// them, works at 0.6, 0.8 or 0.85 of that rate with one, two or three workgroups resident, and writes and reads back
+// n partials (128 KiB at a CU's share of HBM, 139 rows' worth of MFMA time).
+int gram_f32_parts(int64_t tiles, int64_t K, int cus) {
+    if (cus <= 0) return 1;
+    double best = 0.0;
+    int best_parts = 1;
+    for (int parts = 1; parts <= 16 && (parts == 1 || parts * 64 <= K); ++parts) {
+        const int64_t n = (tiles * parts + cus - 1) / cus;
+        const double rate = n == 1 ? 0.6 : n == 2 ? 0.8 : 0.85;
+        const double cost = static_cast<double>(n) / parts / rate + (parts > 1 ? 139.0 * n / K : 0.0);
+        if (parts == 1 || cost < best - 1e-9) {
+            best = cost;
+            best_parts = parts;
+        }
+    }
+    return best_parts;
+}
+
+size_t gram_f32_workspace(int64_t tiles, int parts) {
+    return parts > 1 ? static_cast<size_t>(tiles) * parts * kGramPartial * sizeof(f32x4) : 0;
+}
+
+bool f32_symmetric(const float* C, const void* A, const void* B, const void* B2, int64_t M, int64_t N, int64_t lda,
+                   int64_t ldb, int64_t ldc) {
+    return A == B && !B2 && lda == ldb && M == N && ldc % 4 == 0 && reinterpret_cast<uintptr_t>(C) % 16 == 0;
+}
+
+int64_t f32_sym_tiles(int64_t M) {
+    const int64_t tm = (M + kBM - 1) / kBM;
+    return tm * (tm + 1) / 2;
+}
+
 }  // namespace
 
 extern "C" {
 
 size_t qsrt_gemm_tn_workspace_bytes(const float* C, const void* A, const void* B, int64_t M, int64_t N, int64_t K,
                                     int64_t lda, int64_t ldb, int64_t ldc, int dtype) {
-    if (dtype != 1 || M <= 0 || N <= 0 || K <= 0) return 0;
+    if (M <= 0 || N <= 0 || K <= 0) return 0;
+    if (dtype == 0 && f32_symmetric(C, A, B, nullptr, M, N, lda, ldb, ldc)) {
+        const int64_t tiles = f32_sym_tiles(M);
+        return gram_f32_workspace(tiles, gram_f32_parts(tiles, K, device_cus()));
+    }
+    if (dtype != 1) return 0;
     const bool sym = bf16_symmetric(C, A, B, M, N, lda, ldb, ldc);
     return bf16_plan(bf16_tiles(sym, M, N), (K + kBK16 - 1) / kBK16, device_cus()).workspace_bytes();
 }
@@ -546,6 +707,29 @@ int qsrt_gemm_tn_ws(float* C, const void* A, const void* B, const void* B2, int6
         if (lda % 4 || ldb % 4 || reinterpret_cast<uintptr_t>(A) % 16 || reinterpret_cast<uintptr_t>(B) % 16 ||
             (B2 && reinterpret_cast<uintptr_t>(B2) % 16))
             return qsrt::fail(qsrt::kBadArgument, "f32 operands must be 16-byte aligned with lda, ldb multiples of 4");
+        if (f32_symmetric(C, A, B, B2, M, N, lda, ldb, ldc)) {
+            const int64_t sym = f32_sym_tiles(M);
+            int parts = gram_f32_parts(sym, K, device_cus());
+            if (!workspace || workspace_bytes < gram_f32_workspace(sym, parts) ||
+                reinterpret_cast<uintptr_t>(workspace) % 16)
+                parts = 1;  // no room for the partials: every tile whole
+            if (sym * parts > 0x7fffffff / 4) return qsrt::fail(qsrt::kBadArgument, "GEMM too large for one launch");
+            const int ti = static_cast<int>((M + kBM - 1) / kBM), n = static_cast<int>(sym);
+            auto* ws = static_cast<f32x4*>(workspace);
+            const auto* x = static_cast<const float*>(A);
+            if (parts == 1) {
+                hipLaunchKernelGGL(gram_f32_kernel<false>, dim3(static_cast<unsigned>(n)), dim3(kThreads), 0, stream, C,
+                                   x, M, K, lda, ldc, alpha, ti, n, 1, nullptr);
+            } else {
+                hipLaunchKernelGGL(gram_f32_kernel<true>, dim3(static_cast<unsigned>(n * parts)), dim3(kThreads), 0,
+                                   stream, C, x, M, K, lda, ldc, alpha, ti, n, parts, ws);
+                QSRT_HIP_TRY(hipGetLastError());
+                hipLaunchKernelGGL(gram_f32_fixup, dim3(static_cast<unsigned>(4 * n)), dim3(kThreads), 0, stream, C, M,
+                                   ldc, alpha, ti, n, parts, ws);
+            }
+            QSRT_HIP_TRY(hipGetLastError());
+            return qsrt::kOk;
+        }
         hipLaunchKernelGGL(gemm_tn_f32_kernel, dim3(static_cast<unsigned>(tiles)), dim3(kThreads), 0, stream, C,
                            static_cast<const float*>(A), static_cast<const float*>(B), static_cast<const float*>(B2),
                            M, N, K, lda, ldb, ldc, alpha, tiles_n);

@@ -77,6 +77,32 @@ def test_bf16_gram_matches_float64(n, k):
     assert _rel(Hf.cpu().double().numpy(), x64.T @ x64) < 1e-5
 
 
+@pytest.mark.parametrize("n,k", [(5, 128), (64, 129), (1000, 4), (1000, 383), (8192, 256), (4096, 644), (16384, 130)])
+def test_f32_gram_matches_float64(n, k):
+    """FP32 Gram: tiles on and above the diagonal and their mirror, whole or
+    in K ranges (the tall ones), at tile edges, into a non-zero H; the same
+    from call to call, and without a workspace equal to FP32 rounding."""
+
+    print(f"[gemm] f32 gram n{n} k{k}", file=sys.stderr, flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(n + k)
+    X = torch.randn(n, k, device="cuda", generator=gen)
+    H0 = torch.randn(k, k, device="cuda", generator=gen)
+    want = H0.double() + X.double().T @ X.double() / n
+    # relative to the largest entry, as everywhere here: sums of n products of standard normals, each rounding 2^-24
+    tol = max(1e-6, 2.0**-24 * n**0.5)
+    H = H0.clone()
+    gemm.gram_(H, X, alpha=1.0 / n)
+    assert (H.double() - want).abs().max().item() <= tol * want.abs().max().item()
+    again = H0.clone()
+    gemm.gram_(again, X, alpha=1.0 / n)
+    assert torch.equal(H, again)
+    if k % 4 == 0:  # the leading dimensions the C entry takes as they are
+        whole = H0.clone()
+        _native.check(_native.lib().qsrt_gemm_tn(whole.data_ptr(), X.data_ptr(), X.data_ptr(), None, k, k, n, k, k, k,
+                                                 1.0 / n, 0, _native.stream_handle(X.device)), "qsrt_gemm_tn")
+        assert (whole - H).abs().max().item() <= 2 * tol * want.abs().max().item()
+
+
 def test_bf16_gram_full_size_matches_float64():
     """The Hessian capture at the config-4 shape: 16,384 bf16 rows x 7168
     channels.  Reference: the float64 product on the device (rocBLAS DGEMM),
