@@ -175,8 +175,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3))) v
 // off-diagonal tiles also add their transpose (float4 stores along m).
 // One workgroup per CU (the LDS buffers take 144 KiB), so a tile count that
 // is not a multiple of the CU count leaves CUs idle in the last round (the
-// 406 Gram tiles of 7168 channels: 150 tiles in a second round on 256 CUs);
-// given a workspace, those tiles are split along K (bf16_plan below).
+// 406 Gram tiles of 7168 channels: 150 tiles in a second round on 256 CUs;
+// the 36 of 2048 channels: 36 in all);
+// given a workspace, those tiles are split along K where it pays (bf16_plan
+// below).
 constexpr int kT16 = 256;
 constexpr int kBK16 = 64;
 constexpr int kRow16 = kT16 + 32;  // LDS row: 256 columns + 32 pad (bf16) = 576 B
@@ -463,11 +465,12 @@ __global__ __launch_bounds__(kThreads16) void gemm_tn_bf16_fixup(float* __restri
     bf16_epilogue<SYM, 1>(C, acc, i, M, N, ldc, alpha, tm, tn, t);
 }
 
-// Launch plan of the bf16 path: `tiles` tiles on `cus` compute units.  A last round that would leave CUs
-// idle is split along K into `parts` ranges, chosen to minimise (rounds of ranges) / parts + 0.09 x
-// (ranges per CU) in units of one tile's time: the first term is the split round's length, the second the
-// cost of writing and re-reading each range's partial (fitted on MI355X to the Gram of a 16384 x 7168
-// operand at 2, 3, 4, 5 and 8 parts; 3 parts there, 8 for the 28 x 28 tiles of the full product).
+// Launch plan of the bf16 path: `tiles` tiles on `cus` compute units.  A last (or only) round of `sk` tiles that would
+// leave CUs idle is split along K into `parts` ranges where that is faster.  Microseconds, fitted to Grams of 256 to
+// 7168 channels and 171 to 16,384 rows at 1 to 64 parts: a stage of 64 rows takes 1.62; whole tiles add their C
+// traffic at the end; a range writes a partial of 256 KiB that the fixup reads, and the fixup is a launch of its own.
+//   16384 x 7168 (sk 150): whole 1023 us, 3 parts 878, 5 867, 8 903      171 x 7168: whole 82, 2 parts 136, 3 146
+//   16384 x 2048 (sk 36):  whole 413, 7 parts 97, 14 112                 4096 x 7168: whole 269, 3 parts 316
 struct Bf16Plan {
     int64_t tiles = 0, dp = 0, sk = 0;
     int parts = 1;
@@ -477,13 +480,14 @@ struct Bf16Plan {
 Bf16Plan bf16_plan(int64_t tiles, int64_t stages, int cus) {
     Bf16Plan p;
     p.tiles = p.dp = tiles;
-    if (cus <= 0 || tiles <= cus || tiles % cus == 0 || stages < 2) return p;
+    if (cus <= 0 || tiles % cus == 0 || stages < 2) return p;
     const int64_t sk = tiles % cus;
-    double best = 1.0;  // an unsplit last round: one tile's time
+    const double stage = 1.62 * static_cast<double>(stages), tail = static_cast<double>(sk);
+    double best = stage + 22.0 + 0.07 * tail;
     int best_parts = 1;
-    for (int parts = 2; parts <= 8 && parts <= stages; ++parts) {
-        const double rounds = static_cast<double>((sk * parts + cus - 1) / cus);
-        const double cost = rounds / parts + 0.09 * static_cast<double>(sk * parts) / cus;
+    for (int parts = 2; parts <= 32 && parts <= stages; ++parts) {
+        const double ranges = static_cast<double>((sk * parts + cus - 1) / cus);
+        const double cost = ranges * stage / parts + 0.1 * tail * parts + 13.0 + 0.1 * tail;
         if (cost < best - 1e-9) {
             best = cost;
             best_parts = parts;

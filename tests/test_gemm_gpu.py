@@ -103,6 +103,27 @@ def test_f32_gram_matches_float64(n, k):
         assert (whole - H).abs().max().item() <= 2 * tol * want.abs().max().item()
 
 
+@pytest.mark.parametrize("n,k", [(130, 7), (129, 300), (8192, 256), (8191, 40), (4096, 1030), (300, 4200), (16384, 2056)])
+def test_bf16_gram_with_fewer_tiles_than_units(n, k):
+    """Tile counts below the compute units': K ranges of every tile (or whole
+    tiles, at few rows), ragged rows and channels, into a non-zero H; equal
+    to the whole tiles to FP32 rounding and the same from call to call."""
+
+    print(f"[gemm] bf16 small gram n{n} k{k}", file=sys.stderr, flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(3 * n + k)
+    X = torch.randn(n, k, device="cuda", generator=gen).bfloat16()
+    H0 = torch.randn(k, k, device="cuda", generator=gen)
+    H0 = H0 + H0.T
+    want = H0.double() + X.double().T @ X.double() / n
+    tol = max(1e-6, 2.0**-24 * n**0.5)  # FP32 sums of n exact products, relative to the largest entry
+    H = H0.clone()
+    gemm.gram_(H, X, alpha=1.0 / n)
+    assert (H.double() - want).abs().max().item() <= tol * want.abs().max().item()
+    again = H0.clone()
+    gemm.gram_(again, X, alpha=1.0 / n)
+    assert torch.equal(H, again)
+
+
 def test_bf16_gram_full_size_matches_float64():
     """The Hessian capture at the config-4 shape: 16,384 bf16 rows x 7168
     channels.  Reference: the float64 product on the device (rocBLAS DGEMM),
