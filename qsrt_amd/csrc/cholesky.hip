@@ -10,19 +10,24 @@
 // also returns the block's inverse so that the panel solve
 // L21 = A21 L11^-T becomes one more DGEMM.
 //
-// Block of nb <= 128 rows, 1024 threads: thread (ti, tj) = (t / 32, t % 32) keeps the 4 x 4 sub-block of
-// rows 4 ti .. 4 ti + 3 and columns 4 tj .. 4 tj + 3 in registers for the whole call,
-// so each elimination step is a branch-free outer-product update from one published column:
-//   Cholesky  step k: the owners of column k publish it below the diagonal (zeros at and above it) and the
-//             pivot a_kk; every thread computes d = sqrt(a_kk), l_ik = a_ik * (1 / d) (the reciprocal
-//             multiply of LAPACK's dpotf2) for its rows and columns and does a_ij -= l_ik l_jk (fma); the
-//             owners of column k then keep d and l_ik.  Entries above the diagonal are updated too and
-//             never read.
-//   inverse   X = L11^-1, X = I to start; step k: the owners of row k divide it by l_kk and publish it,
-//             the owners of column k of L11 publish it below the diagonal, and every thread does
-//             x_ic -= l_ik x_kc (fma).
-// A wave whose rows all lie above row k has nothing left to update and skips the step.  Two barriers
-// per step of each pass.  One workgroup per matrix of a batch.
+// Block of nb <= 128 rows, 16 waves.  In the factorisation wave w keeps columns 8 w .. 8 w + 7 of the block in
+// registers, a lane two rows (l and l + 64); in the inverse X = L11^-1 it keeps rows 8 w .. 8 w + 7, a lane two
+// columns.  A panel of eight columns then belongs to one wave, and so do eight rows of X:
+//   factor    step k: the pivot a_kk is read from its lane, d = sqrt(a_kk), l_ik = a_ik * (1 / d) (the reciprocal
+//             multiply of LAPACK's dpotf2) and a_ij -= l_ik l_jk (fma) for the panel's later columns, l_jk read from
+//             lane j: no barrier inside a panel.  The panel goes to LDS.
+//   update    every later wave: a_ij -= l_ik l_jk for the panel's eight k, ascending.
+//   solve     the panel's wave, one panel later: its rows of X, x_kc / l_kk and x_ic -= l_ik x_kc, no barrier either.
+// One round p is [wave p factors, wave p - 1 solves], barrier, [later waves update from both]: one barrier per eight
+// columns, the solve in the shadow of the factor, and each element meets its fmas in the order k = 0, 1, ... of the
+// plain right-looking algorithm.
+//
+// What bounds it is the chain of pivots, 128 square roots and reciprocals one after the other: 560 cycles a column,
+// so 4500 of the 6600 (late) to 8400 (early) cycles of a round, the rest being the update that the next panel's wave
+// has to finish first, among the LDS reads of the others.  That wave therefore runs at raised priority and leaves its
+// rows of X for the round after (66 us without, 60 us with).  With one barrier per column, all 16 waves in each, and
+// each evaluating the root, a block of 128 rows took 237 us between two events, of 64 rows 128 us and of 16 rows
+// 40 us; it takes 60, 37 and 19 us, with the same bits.  One workgroup per matrix of a batch.
 
 #include "common.h"
 #include "qsrt_amd.h"
@@ -30,10 +35,55 @@
 namespace {
 
 constexpr int kMaxNb = 128;
-constexpr int kSub = 4;                              // rows and columns of a thread's sub-block
-constexpr int kGroups = kMaxNb / kSub;               // sub-blocks per row of the block (32)
-constexpr int kThreadsChol = kGroups * kGroups;      // 1024
-constexpr int kRowGroupsPerWave = 64 / kGroups;      // 2
+constexpr int kPanel = 8;                           // columns of a panel, rows of X of a wave
+constexpr int kPanels = kMaxNb / kPanel;            // 16
+constexpr int kThreadsChol = 64 * kPanels;          // a wave per panel
+constexpr int kLdL = kMaxNb + 2;                    // doubles per column of L in LDS: 16-byte aligned, and the final
+                                                    // transposed read meets a bank 4 times instead of 64
+
+struct CholShared {
+    double L[kMaxNb * kLdL];         // column-major: l_ik at k * kLdL + i
+    double X[2][kPanel * kMaxNb];    // eight rows of X, two panels in turn
+    int failed[kPanels];             // 1 + the step whose pivot is not positive, per panel
+};
+
+__device__ __forceinline__ double lane_value(double v, int lane) {
+    const int lo = __builtin_amdgcn_readlane(__double2loint(v), lane);
+    const int hi = __builtin_amdgcn_readlane(__double2hiint(v), lane);
+    return __hiloint2double(hi, lo);
+}
+
+// Factors panel p from its wave's registers; R is the register row that holds rows 8 p .. (rows l for p < 8, l + 64
+// from there on, where the rows l lie above the panel and are left out).
+template <int R>
+__device__ __forceinline__ void factor_panel(double (&a)[2][kPanel], int p, int nb, CholShared& sh) {
+    const int lane = static_cast<int>(threadIdx.x) & 63;
+    const int k0 = kPanel * p, lane0 = k0 & 63;
+#pragma unroll
+    for (int c = 0; c < kPanel; ++c) {
+        const int k = k0 + c;
+        if (k >= nb) break;
+        const double piv = lane_value(a[R][c], lane0 + c);
+        if (!(piv > 0.0)) {
+            if (lane == 0) sh.failed[p] = k + 1;
+            return;
+        }
+        const double d = sqrt(piv), rd = 1.0 / d;
+#pragma unroll
+        for (int r = R; r < 2; ++r) a[r][c] *= rd;
+#pragma unroll
+        for (int j = c + 1; j < kPanel; ++j) {
+            const double lj = lane_value(a[R][c], lane0 + j);
+#pragma unroll
+            for (int r = R; r < 2; ++r) a[r][j] = fma(-a[r][c], lj, a[r][j]);
+        }
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            const int i = lane + 64 * r;
+            sh.L[k * kLdL + i] = i > k ? a[r][c] : i == k ? d : 0.0;
+        }
+    }
+}
 
 // The nb x nb diagonal block at (j0, j0) of matrix blockIdx.x (leading dimension n, batch stride
 // `stride`): its lower triangle is read, the factor L11 is written over it with zeros above the
@@ -44,136 +94,122 @@ __global__ __launch_bounds__(kThreadsChol) void chol_diag_block_f64_kernel(doubl
                                                                            int64_t stride, int64_t j0, int nb,
                                                                            double* __restrict__ inv,
                                                                            int32_t* __restrict__ info) {
-    __shared__ double colv[kMaxNb];  // the published column (Cholesky: a_ik; inverse: l_ik), zero at i <= k
-    __shared__ double rowv[kMaxNb];  // inverse: the published row k of X
-    __shared__ double diag[kMaxNb];  // l_kk
-    __shared__ double pivot;
+    __shared__ __attribute__((aligned(16))) CholShared sh;
     const int t = static_cast<int>(threadIdx.x);
-    const int ti = t / kGroups, tj = t % kGroups;
-    const int i0 = kSub * ti, c0 = kSub * tj;
-    const int wave_last_row = kSub * ((t >> 6) * kRowGroupsPerWave + kRowGroupsPerWave) - 1;  // of this wave
+    const int lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int panels = (nb + kPanel - 1) / kPanel;
     double* M = A + static_cast<int64_t>(blockIdx.x) * stride + j0 * n + j0;
     double* Xo = inv + static_cast<int64_t>(blockIdx.x) * nb * nb;
 
-    double a[kSub][kSub];
+    // Row-major lines in, columns out: through LDS, as the other way a load would touch 64 lines.
+    double in[kMaxNb * kMaxNb / kThreadsChol];
 #pragma unroll
-    for (int r = 0; r < kSub; ++r)
-#pragma unroll
-        for (int c = 0; c < kSub; ++c) {
-            const int i = i0 + r, j = c0 + c;
-            a[r][c] = i < nb && j <= i ? M[static_cast<int64_t>(i) * n + j] : 0.0;
-        }
-
-    int failed = 0;
-    for (int k = 0; k < nb; ++k) {
-        const int kc = k % kSub;
-        if (tj == k / kSub) {
-#pragma unroll
-            for (int c = 0; c < kSub; ++c)
-                if (c == kc) {  // uniform: k is the same for every thread
-#pragma unroll
-                    for (int r = 0; r < kSub; ++r) {
-                        const int i = i0 + r;
-                        colv[i] = i > k ? a[r][c] : 0.0;
-                        if (i == k) pivot = a[r][c];
-                    }
-                }
-        }
-        __syncthreads();
-        const double piv = pivot;  // the same value for every thread: the branch is uniform
-        if (!(piv > 0.0)) {
-            failed = k + 1;
-            break;
-        }
-        if (wave_last_row >= k) {  // the wave holding row k finalises a_kk
-            const double d = sqrt(piv), rd = 1.0 / d;
-            double li[kSub], lj[kSub];
-#pragma unroll
-            for (int q = 0; q < kSub; ++q) {
-                li[q] = colv[i0 + q] * rd;
-                lj[q] = colv[c0 + q] * rd;
-            }
-#pragma unroll
-            for (int r = 0; r < kSub; ++r)
-#pragma unroll
-                for (int c = 0; c < kSub; ++c) a[r][c] = fma(-li[r], lj[c], a[r][c]);
-            if (tj == k / kSub) {
-#pragma unroll
-                for (int c = 0; c < kSub; ++c)
-                    if (c == kc) {
-#pragma unroll
-                        for (int r = 0; r < kSub; ++r) {
-                            const int i = i0 + r;
-                            a[r][c] = i == k ? d : i > k ? li[r] : a[r][c];
-                        }
-                    }
-            }
-        }
-        __syncthreads();
-    }
-    if (failed) {
-        if (t == 0) atomicCAS(info + blockIdx.x, 0, static_cast<int32_t>(j0 + failed));
-        return;
+    for (int e = 0; e < kMaxNb * kMaxNb / kThreadsChol; ++e) {
+        const int i = w + kPanels * (e >> 1), j = lane + 64 * (e & 1);
+        in[e] = i < nb && j <= i ? M[static_cast<int64_t>(i) * n + j] : 0.0;
     }
 #pragma unroll
-    for (int r = 0; r < kSub; ++r)
-#pragma unroll
-        for (int c = 0; c < kSub; ++c) {
-            const int i = i0 + r, j = c0 + c;
-            if (i < nb && j < nb) M[static_cast<int64_t>(i) * n + j] = j <= i ? a[r][c] : 0.0;
-            if (i == j && i < nb) diag[i] = a[r][c];
-        }
-
-    double x[kSub][kSub];
-#pragma unroll
-    for (int r = 0; r < kSub; ++r)
-#pragma unroll
-        for (int c = 0; c < kSub; ++c) x[r][c] = i0 + r == c0 + c && i0 + r < nb ? 1.0 : 0.0;
+    for (int e = 0; e < kMaxNb * kMaxNb / kThreadsChol; ++e)
+        sh.L[(lane + 64 * (e & 1)) * kLdL + w + kPanels * (e >> 1)] = in[e];
+    if (t < kPanels) sh.failed[t] = 0;
     __syncthreads();
-    for (int k = 0; k < nb; ++k) {
-        const int kc = k % kSub;
-        if (ti == k / kSub) {
-            const double lkk = diag[k];
+    double a[2][kPanel], x[kPanel][2];
 #pragma unroll
-            for (int r = 0; r < kSub; ++r)
-                if (r == kc) {  // uniform
+    for (int c = 0; c < kPanel; ++c)
 #pragma unroll
-                    for (int c = 0; c < kSub; ++c) {
-                        x[r][c] = x[r][c] / lkk;
-                        rowv[c0 + c] = x[r][c];
-                    }
-                }
+        for (int r = 0; r < 2; ++r) {
+            a[r][c] = sh.L[(kPanel * w + c) * kLdL + lane + 64 * r];
+            x[c][r] = kPanel * w + c == lane + 64 * r ? 1.0 : 0.0;
         }
-        if (tj == k / kSub) {
-#pragma unroll
-            for (int c = 0; c < kSub; ++c)
-                if (c == kc) {
-#pragma unroll
-                    for (int r = 0; r < kSub; ++r) colv[i0 + r] = i0 + r > k ? a[r][c] : 0.0;
-                }
+
+    // Nothing is overwritten early: a wave writes only columns of L that it alone has read before, and the rows of X
+    // of panel p (written in round p + 1) make room for those of panel p + 2 in round p + 3, after the barrier of round
+    // p + 2, which their readers reach last, or by the one wave that is later than that, p + 2 itself.
+    for (int p = 0; p <= panels; ++p) {
+        int own = w;  // the compiler knows p == w inside and would keep every predicate of the panel over the loop
+        asm volatile("" : "+s"(own));
+        if (w == p && p < panels) {
+            if (p < kPanels / 2)
+                factor_panel<0>(a, own, nb, sh);
+            else
+                factor_panel<1>(a, own, nb, sh);
         }
-        __syncthreads();
-        if (wave_last_row > k) {
-            double li[kSub], xk[kSub];
+        if (w == p - 1) {  // rows 8 w ..: their columns of L are this wave's own, written in the round before
+            const int k0 = kPanel * own;
+            double* row = sh.X[own & 1];
 #pragma unroll
-            for (int q = 0; q < kSub; ++q) {
-                li[q] = colv[i0 + q];
-                xk[q] = rowv[c0 + q];
+            for (int c = 0; c < kPanel; ++c) {
+                if (k0 + c >= nb) break;
+                const double lkk = sh.L[(k0 + c) * kLdL + k0 + c];
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    x[c][q] = x[c][q] / lkk;
+                    row[c * kMaxNb + lane + 64 * q] = x[c][q];
+                }
+#pragma unroll
+                for (int i = c + 1; i < kPanel; ++i) {
+                    const double li = sh.L[(k0 + c) * kLdL + k0 + i];
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) x[i][q] = fma(-li, x[c][q], x[i][q]);
+                }
             }
-#pragma unroll
-            for (int r = 0; r < kSub; ++r)
-#pragma unroll
-                for (int c = 0; c < kSub; ++c) x[r][c] = fma(-li[r], xk[c], x[r][c]);
         }
+        __builtin_amdgcn_s_setprio(0);
         __syncthreads();
+        if (p < panels) {
+            if (const int failed = sh.failed[p]) {  // the same word for every thread: uniform
+                if (t == 0) atomicCAS(info + blockIdx.x, 0, static_cast<int32_t>(j0 + failed));
+                return;
+            }
+            if (w == p + 1) __builtin_amdgcn_s_setprio(3);  // the chain goes through this wave
+            if (w > p) {
+#pragma unroll 2
+                for (int k = 0; k < kPanel; ++k) {
+                    const double* l = sh.L + (kPanel * p + k) * kLdL;
+                    double lj[kPanel];
+#pragma unroll
+                    for (int c = 0; c < kPanel; ++c) lj[c] = l[kPanel * w + c];
+                    if (w < kPanels / 2) {  // rows l reach below the diagonal of these columns
+                        const double li = l[lane];
+#pragma unroll
+                        for (int c = 0; c < kPanel; ++c) a[0][c] = fma(-li, lj[c], a[0][c]);
+                    }
+                    const double li = l[lane + 64];
+#pragma unroll
+                    for (int c = 0; c < kPanel; ++c) a[1][c] = fma(-li, lj[c], a[1][c]);
+                }
+            }
+        }
+        // Rows of X of the panels before p; the wave that factors next has its factor to get on with and takes the
+        // last two together a round later (rows p - 2 are overwritten by its own solve at the earliest).
+        const int first = w == p + 1 ? p : w == p && p > 1 ? p - 2 : p - 1;
+        for (int s = first < 0 ? 0 : first; s < p && w >= p; ++s) {
+            const double* row = sh.X[s & 1];
+#pragma unroll 2
+            for (int k = 0; k < kPanel; ++k) {
+                const double* l = sh.L + (kPanel * s + k) * kLdL + kPanel * w;
+                const double x0 = row[k * kMaxNb + lane], x1 = row[k * kMaxNb + lane + 64];
+#pragma unroll
+                for (int i = 0; i < kPanel; ++i) {
+                    const double li = l[i];
+                    x[i][0] = fma(-li, x0, x[i][0]);
+                    x[i][1] = fma(-li, x1, x[i][1]);
+                }
+            }
+        }
     }
 #pragma unroll
-    for (int r = 0; r < kSub; ++r)
+    for (int c = 0; c < kPanel; ++c)
 #pragma unroll
-        for (int c = 0; c < kSub; ++c) {
-            const int i = i0 + r, j = c0 + c;
-            if (i < nb && j < nb) Xo[i * nb + j] = j <= i ? x[r][c] : 0.0;
+        for (int q = 0; q < 2; ++q) {
+            const int i = kPanel * w + c, j = lane + 64 * q;
+            if (i < nb && j < nb) Xo[i * nb + j] = j <= i ? x[c][q] : 0.0;
         }
+#pragma unroll
+    for (int e = 0; e < kMaxNb * kMaxNb / kThreadsChol; ++e) {
+        const int i = w + kPanels * (e >> 1), j = lane + 64 * (e & 1);
+        if (i < nb && j < nb) M[static_cast<int64_t>(i) * n + j] = sh.L[j * kLdL + i];
+    }
 }
 
 }  // namespace

@@ -87,6 +87,36 @@ def test_diagonal_block_and_its_inverse(nb):
     assert torch.equal(M[outside], A[outside])
 
 
+@pytest.mark.parametrize("nb", [7, 8, 9, 16, 57, 63, 65, 72, 121, 127])
+def test_diagonal_block_at_the_edges_of_its_panels(nb):
+    """Blocks around the eight-column panels and the 64-row halves.  With u = 2^-53 and the diagonal's maximum m,
+    |L L^T - A| <= (nb + 1) u |L||L^T| <= (nb + 1) u m (Cauchy-Schwarz on rows of L), and as much again, with a term
+    to spare, for the product formed here; |L X - I| <= nb u |L||X| for each column solved, likewise twice.  A pivot
+    spoilt in the block's last row is the one that ``info`` names."""
+
+    n, j0 = 140, 6
+    A = _spd(n, 50 + nb)
+    lib = _native.lib()
+
+    def run(M):
+        inv = torch.full((nb, nb), float("nan"), dtype=torch.float64, device=DEV)
+        info = torch.zeros(1, dtype=torch.int32, device=DEV)
+        _native.check(lib.qsrt_chol_diag_block_f64(M.data_ptr(), n, 1, n * n, j0, nb, inv.data_ptr(),
+                                                    info.data_ptr(), _native.stream_handle(DEV)), "chol")
+        torch.cuda.synchronize()
+        return M[j0:j0 + nb, j0:j0 + nb].cpu(), inv.cpu(), int(info)
+
+    L, X, info = run(A.clone())
+    want = A[j0:j0 + nb, j0:j0 + nb].cpu()
+    u = 2.0 ** -53
+    assert info == 0
+    assert torch.equal(L, torch.tril(L)) and torch.equal(X, torch.tril(X))
+    assert (L @ L.T - want).abs().max() <= 2 * (nb + 2) * u * want.diagonal().max()
+    assert ((L @ X - torch.eye(nb, dtype=torch.float64)).abs() <= 2 * (nb + 2) * u * (L.abs() @ X.abs())).all()
+    A[j0 + nb - 1, j0 + nb - 1] = float("nan")
+    assert run(A)[2] == j0 + nb
+
+
 @pytest.mark.parametrize("bad_row", [0, 127, 128, 300])
 def test_info_reports_the_first_indefinite_leading_minor(bad_row):
     n = 400
