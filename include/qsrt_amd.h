@@ -275,7 +275,8 @@ size_t qsrt_gemm_tn_workspace_bytes(const float *C, const void *A, const void *B
  * the last round are split along K where that is faster and their partial
  * products, written to the workspace, are added to C in K order by a second
  * kernel on the same stream (the result is deterministic; it differs from the
- * unsplit sum only by FP32 rounding).  f32 with A == B and no B2 (a Gram):
+ * unsplit sum only by FP32 rounding), or, at few rows, every tile sums its
+ * rows in groups of 64 and needs no workspace.  f32 with A == B and no B2 (a Gram):
  * likewise for its 128 x 128 tiles on and above the diagonal, the only ones
  * computed.  A NULL or short workspace runs every tile whole, as
  * qsrt_gemm_tn does.  Same operator and call sites as qsrt_gemm_tn.

@@ -177,8 +177,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3))) v
 // is not a multiple of the CU count leaves CUs idle in the last round (the
 // 406 Gram tiles of 7168 channels: 150 tiles in a second round on 256 CUs;
 // the 36 of 2048 channels: 36 in all);
-// given a workspace, those tiles are split along K where it pays (bf16_plan
-// below).
+// given a workspace, those tiles are split along K where it pays, or at few
+// rows all tiles run staged (bf16_plan below).
 constexpr int kT16 = 256;
 constexpr int kBK16 = 64;
 constexpr int kRow16 = kT16 + 32;  // LDS row: 256 columns + 32 pad (bf16) = 576 B
@@ -277,8 +277,11 @@ __device__ __forceinline__ int xcd_slot(int q, int n) {
 
 typedef uint16_t Bf16Lds[2][2][kBK16 * kRow16];  // [buffer][operand][k-row, column]
 
-// acc += A[k0 .. k1)^T B[k0 .. k1) over the tile's columns m0 .. m0 + 255 of A and n0 .. n0 + 255 of B
-__device__ __forceinline__ void bf16_mainloop(f32x4 (&acc)[8][4], Bf16Lds& S, const uint16_t* __restrict__ A,
+// acc += A[k0 .. k1)^T B[k0 .. k1) over the tile's columns m0 .. m0 + 255 of A and n0 .. n0 + 255 of B, the 16-row
+// blocks i0 .. i0 + IB - 1 of every wave's 128 x 64 block.  With STAGED (half a block: the registers) the 64 rows of a
+// stage are summed by themselves and then added.
+template <int IB, bool STAGED>
+__device__ __forceinline__ void bf16_mainloop(f32x4 (&acc)[IB][4], int i0, Bf16Lds& S, const uint16_t* __restrict__ A,
                                               const uint16_t* __restrict__ B, int64_t M, int64_t N, int64_t k0,
                                               int64_t k1, int64_t lda, int64_t ldb, int64_t m0, int64_t n0, int t) {
     const int lane = t & 63, wave = t >> 6;
@@ -303,30 +306,55 @@ __device__ __forceinline__ void bf16_mainloop(f32x4 (&acc)[8][4], Bf16Lds& S, co
     __syncthreads();
     for (int64_t s = 0; s < stages; ++s) {
         const int cur = static_cast<int>(s & 1);
+        // Between the two halves of the stage (the other buffer is free since the last barrier): the
+        // next stage goes to LDS and the one after is requested, so the waves' store phases overlap
+        // the second half's MFMAs and the loads have a stage and a half to land.
+        const auto next_stage = [&]() {
+            if (s + 1 < stages) {
+                store_stage(ua, S[cur ^ 1][0], t);
+                store_stage(ub, S[cur ^ 1][1], t);
+            }
+            if (s + 2 < stages) {
+                load_stage(ua, PA, (s + 2) * kBK16, K, lda, spanA, t);
+                load_stage(ub, PB, (s + 2) * kBK16, K, ldb, spanB, t);
+            }
+        };
+        if constexpr (STAGED) {
+            bf16x8 b0[4], b1[4];
 #pragma unroll
-        for (int kk = 0; kk < kBK16; kk += 32) {
-            bf16x8 a[8], b[4];
+            for (int j = 0; j < 4; ++j) {
+                b0[j] = fragment(S[cur][1], 0, wn + 16 * j, lane);
+                b1[j] = fragment(S[cur][1], 32, wn + 16 * j, lane);
+            }
 #pragma unroll
-            for (int i = 0; i < 8; ++i) a[i] = fragment(S[cur][0], kk, wm + 16 * i, lane);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) b[j] = fragment(S[cur][1], kk, wn + 16 * j, lane);
-#pragma unroll
-            for (int i = 0; i < 8; ++i)
+            for (int i = 0; i < IB; ++i) {
+                const bf16x8 a0 = fragment(S[cur][0], 0, wm + 16 * (i0 + i), lane);
+                const bf16x8 a1 = fragment(S[cur][0], 32, wm + 16 * (i0 + i), lane);
+                f32x4 sum[4];
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
-            if (kk == 0) {
-                // Between the two halves of the stage (the other buffer is free since the last barrier): the
-                // next stage goes to LDS and the one after is requested, so the waves' store phases overlap
-                // the second half's MFMAs and the loads have a stage and a half to land.
-                if (s + 1 < stages) {
-                    store_stage(ua, S[cur ^ 1][0], t);
-                    store_stage(ub, S[cur ^ 1][1], t);
-                }
-                if (s + 2 < stages) {
-                    load_stage(ua, PA, (s + 2) * kBK16, K, lda, spanA, t);
-                    load_stage(ub, PB, (s + 2) * kBK16, K, ldb, spanB, t);
-                }
+                    sum[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b0[j], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    sum[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b1[j], sum[j], 0, 0, 0);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc[i][j] += sum[j];
+                if (i == IB / 2 - 1) next_stage();
+            }
+        } else {
+#pragma unroll
+            for (int kk = 0; kk < kBK16; kk += 32) {
+                bf16x8 a[IB], b[4];
+#pragma unroll
+                for (int i = 0; i < IB; ++i) a[i] = fragment(S[cur][0], kk, wm + 16 * (i0 + i), lane);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) b[j] = fragment(S[cur][1], kk, wn + 16 * j, lane);
+#pragma unroll
+                for (int i = 0; i < IB; ++i)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+                if (kk == 0) next_stage();
             }
         }
         __syncthreads();
@@ -402,12 +430,13 @@ __device__ __forceinline__ void bf16_epilogue(float* __restrict__ C, const f32x4
 // so a wave's stores and loads are contiguous.
 constexpr int64_t kPartialVec = 32 * kThreads16;  // f32x4 per partial (256 KiB)
 
-// Workgroups [0, dp) each own a whole tile: order[xcd_slot(b, dp)].  When the tile count is not a multiple
+// Workgroups [0, dp) each own a whole tile: order[xcd_slot(b, dp)] (with STAGED all of them, in two passes over K, one
+// per half of every wave's block: 64 accumulators and the sums of a stage fit the registers, 128 do not).  When the tile count is not a multiple
 // of the CU count, the tiles order[dp .. dp + sk) of the last, partial round are instead split into `parts`
 // K ranges and the workgroups [dp, dp + sk * parts) compute one range each into the workspace, range-major
 // (all first ranges, then all second ranges, ...), so the workgroups resident on one XCD at a time walk the
 // same K range of neighbouring tiles; gemm_tn_bf16_fixup adds the ranges to C in K order.
-template <bool SYM>
+template <bool SYM, bool STAGED>
 __global__ __launch_bounds__(kThreads16) void gemm_tn_bf16_kernel(float* __restrict__ C, const uint16_t* __restrict__ A,
                                                                   const uint16_t* __restrict__ B, int64_t M,
                                                                   int64_t N, int64_t K, int64_t lda, int64_t ldb,
@@ -416,16 +445,31 @@ __global__ __launch_bounds__(kThreads16) void gemm_tn_bf16_kernel(float* __restr
     __shared__ __attribute__((aligned(16))) Bf16Lds S;
     const int b = static_cast<int>(blockIdx.x), t = static_cast<int>(threadIdx.x);
     const int tiles_m = static_cast<int>((M + kT16 - 1) / kT16);
+    int tm = 0, tn = 0;
+    if constexpr (STAGED) {
+        if (!tile_at(xcd_slot(b, dp), tiles_m, tiles_n, SYM, tm, tn)) return;  // not reached: dp is the tile count
+#pragma unroll 1
+        for (int i0 = 0; i0 < 8; i0 += 4) {
+            f32x4 acc[4][4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+            bf16_mainloop<4, true>(acc, i0, S, A, B, M, N, 0, K, lda, ldb, static_cast<int64_t>(tm) * kT16,
+                                   static_cast<int64_t>(tn) * kT16, t);
+            bf16_epilogue<SYM, 4>(C, acc, i0, M, N, ldc, alpha, tm, tn, t);
+        }
+        return;
+    }
     f32x4 acc[8][4];
 #pragma unroll
     for (int i = 0; i < 8; ++i)
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    int tm = 0, tn = 0;
     if (b < dp) {
         if (!tile_at(xcd_slot(b, dp), tiles_m, tiles_n, SYM, tm, tn)) return;  // not reached: dp <= tiles
-        bf16_mainloop(acc, S, A, B, M, N, 0, K, lda, ldb, static_cast<int64_t>(tm) * kT16,
-                      static_cast<int64_t>(tn) * kT16, t);
+        bf16_mainloop<8, false>(acc, 0, S, A, B, M, N, 0, K, lda, ldb, static_cast<int64_t>(tm) * kT16,
+                                static_cast<int64_t>(tn) * kT16, t);
         bf16_epilogue<SYM, 8>(C, acc, 0, M, N, ldc, alpha, tm, tn, t);
         return;
     }
@@ -433,8 +477,8 @@ __global__ __launch_bounds__(kThreads16) void gemm_tn_bf16_kernel(float* __restr
     if (!tile_at(dp + s, tiles_m, tiles_n, SYM, tm, tn)) return;  // not reached
     const int64_t stages = (K + kBK16 - 1) / kBK16;
     const int64_t k0 = stages * part / parts * kBK16, k1 = stages * (part + 1) / parts * kBK16;
-    bf16_mainloop(acc, S, A, B, M, N, k0, k1 < K ? k1 : K, lda, ldb, static_cast<int64_t>(tm) * kT16,
-                  static_cast<int64_t>(tn) * kT16, t);
+    bf16_mainloop<8, false>(acc, 0, S, A, B, M, N, k0, k1 < K ? k1 : K, lda, ldb, static_cast<int64_t>(tm) * kT16,
+                            static_cast<int64_t>(tn) * kT16, t);
     f32x4* w = ws + static_cast<int64_t>(part * sk + s) * kPartialVec;
 #pragma unroll
     for (int i = 0; i < 8; ++i)
@@ -465,15 +509,24 @@ __global__ __launch_bounds__(kThreads16) void gemm_tn_bf16_fixup(float* __restri
     bf16_epilogue<SYM, 1>(C, acc, i, M, N, ldc, alpha, tm, tn, t);
 }
 
-// Launch plan of the bf16 path: `tiles` tiles on `cus` compute units.  A last (or only) round of `sk` tiles that would
-// leave CUs idle is split along K into `parts` ranges where that is faster.  Microseconds, fitted to Grams of 256 to
-// 7168 channels and 171 to 16,384 rows at 1 to 64 parts: a stage of 64 rows takes 1.62; whole tiles add their C
-// traffic at the end; a range writes a partial of 256 KiB that the fixup reads, and the fixup is a launch of its own.
-//   16384 x 7168 (sk 150): whole 1023 us, 3 parts 878, 5 867, 8 903      171 x 7168: whole 82, 2 parts 136, 3 146
-//   16384 x 2048 (sk 36):  whole 413, 7 parts 97, 14 112                 4096 x 7168: whole 269, 3 parts 316
+// Launch plan of the bf16 path: `tiles` tiles on `cus` compute units, the `sk` tiles of a last (or only) round that would
+// leave CUs idle.  Times in microseconds, a stage of 64 rows at 1.62; a range writes a partial of 256 KiB that the fixup
+// reads, and the fixup is a launch of its own.
+//
+// A round behind whole ones is split into the `parts` that minimise (rounds of ranges) / parts + 0.09 x (ranges per CU),
+// unless at few rows the staged kernel gains more from having no partials than it loses by its second pass over K (2.6 a
+// stage).  Unsplit tiles of the plain kernel would be faster still there, but their sums are longer than the ranges':
+// the error against float64 (2-norm) of 171 x 7168 is 7.0e-8 whole, 6.4e-8 in ranges, 5.4e-8 staged.
+//   7168 (sk 150):  171 rows: 3 parts 145 us, staged 89, whole 81      1024: 182, 149, 121      2048: 225, 231, 171
+//                   4096: 314, 407, 296      16384: 3 parts 866, 5 872, 8 944, staged 1472, whole 934
+//   9216 (sk 154):  171 rows: 3 parts 218 us, staged 191      1000: 267, 282
+//   5888 (sk 20):   171 rows: 3 parts 67 us, staged 83        640: 8 parts 84, staged 117
+// An only round is split where the fitted times say so (256 to 5120 channels, 171 to 16,384 rows, 1 to 64 parts):
+//   16384 x 2048 (sk 36): whole 413 us, 7 parts 97, 14 112      300 x 2048: whole kept
 struct Bf16Plan {
     int64_t tiles = 0, dp = 0, sk = 0;
     int parts = 1;
+    bool staged = false;  // whole tiles that sum each stage by itself
     size_t workspace_bytes() const { return sk ? static_cast<size_t>(sk * parts) * kPartialVec * sizeof(f32x4) : 0; }
 };
 
@@ -481,16 +534,32 @@ Bf16Plan bf16_plan(int64_t tiles, int64_t stages, int cus) {
     Bf16Plan p;
     p.tiles = p.dp = tiles;
     if (cus <= 0 || tiles % cus == 0 || stages < 2) return p;
-    const int64_t sk = tiles % cus;
+    const int64_t sk = tiles % cus, rounds = tiles / cus;
     const double stage = 1.62 * static_cast<double>(stages), tail = static_cast<double>(sk);
-    double best = stage + 22.0 + 0.07 * tail;
     int best_parts = 1;
-    for (int parts = 2; parts <= 32 && parts <= stages; ++parts) {
-        const double ranges = static_cast<double>((sk * parts + cus - 1) / cus);
-        const double cost = ranges * stage / parts + 0.1 * tail * parts + 13.0 + 0.1 * tail;
-        if (cost < best - 1e-9) {
-            best = cost;
-            best_parts = parts;
+    if (rounds) {
+        double best = 1.0;  // an unsplit last round: one tile's time
+        for (int parts = 2; parts <= 8 && parts <= stages; ++parts) {
+            const double ranges = static_cast<double>((sk * parts + cus - 1) / cus);
+            const double cost = ranges / parts + 0.09 * static_cast<double>(sk * parts) / cus;
+            if (cost < best - 1e-9) {
+                best = cost;
+                best_parts = parts;
+            }
+        }
+        const double ranges = static_cast<double>((sk * best_parts + cus - 1) / cus), full = static_cast<double>(rounds);
+        const double split = full * stage + ranges * stage / best_parts + 0.107 * tail * best_parts + 0.27 * tail + 8.0;
+        p.staged = best_parts > 1 && (full + 1.0) * 2.6 * static_cast<double>(stages) + 0.07 * tail + 42.0 < split;
+        if (p.staged) return p;
+    } else {
+        double best = stage + 22.0 + 0.07 * tail;
+        for (int parts = 2; parts <= 32 && parts <= stages; ++parts) {
+            const double ranges = static_cast<double>((sk * parts + cus - 1) / cus);
+            const double cost = ranges * stage / parts + 0.1 * tail * parts + 13.0 + 0.1 * tail;
+            if (cost < best - 1e-9) {
+                best = cost;
+                best_parts = parts;
+            }
         }
     }
     if (best_parts == 1) return p;
@@ -678,25 +747,10 @@ int64_t f32_sym_tiles(int64_t M) {
     return tm * (tm + 1) / 2;
 }
 
-}  // namespace
-
-extern "C" {
-
-size_t qsrt_gemm_tn_workspace_bytes(const float* C, const void* A, const void* B, int64_t M, int64_t N, int64_t K,
-                                    int64_t lda, int64_t ldb, int64_t ldc, int dtype) {
-    if (M <= 0 || N <= 0 || K <= 0) return 0;
-    if (dtype == 0 && f32_symmetric(C, A, B, nullptr, M, N, lda, ldb, ldc)) {
-        const int64_t tiles = f32_sym_tiles(M);
-        return gram_f32_workspace(tiles, gram_f32_parts(tiles, K, device_cus()));
-    }
-    if (dtype != 1) return 0;
-    const bool sym = bf16_symmetric(C, A, B, M, N, lda, ldb, ldc);
-    return bf16_plan(bf16_tiles(sym, M, N), (K + kBK16 - 1) / kBK16, device_cus()).workspace_bytes();
-}
-
-int qsrt_gemm_tn_ws(float* C, const void* A, const void* B, const void* B2, int64_t M, int64_t N, int64_t K,
-                    int64_t lda, int64_t ldb, int64_t ldc, float alpha, int dtype, void* workspace,
-                    size_t workspace_bytes, void* stream_handle) {
+// `planned`: the last round as bf16_plan has it; otherwise every bf16 tile runs whole in the plain kernel.
+int gemm_tn(float* C, const void* A, const void* B, const void* B2, int64_t M, int64_t N, int64_t K, int64_t lda,
+            int64_t ldb, int64_t ldc, float alpha, int dtype, bool planned, void* workspace, size_t workspace_bytes,
+            void* stream_handle) {
     hipStream_t stream = static_cast<hipStream_t>(stream_handle);
     if (dtype != 0 && dtype != 1) return qsrt::fail(qsrt::kBadArgument, "dtype must be 0 (f32) or 1 (bf16)");
     if (M < 0 || N < 0 || K < 0) return qsrt::fail(qsrt::kBadArgument, "negative GEMM extent");
@@ -756,17 +810,16 @@ int qsrt_gemm_tn_ws(float* C, const void* A, const void* B, const void* B2, int6
         plan.sk = 0;
         plan.parts = 1;
     }
+    plan.staged = plan.staged && planned;
     const unsigned grid = static_cast<unsigned>(plan.dp + plan.sk * plan.parts);
     auto* ws = static_cast<f32x4*>(workspace);
     const auto* a = static_cast<const uint16_t*>(A);
     const auto* b = static_cast<const uint16_t*>(B);
     const int dp = static_cast<int>(plan.dp), sk = static_cast<int>(plan.sk), ti = static_cast<int>(tn);
-    if (sym)
-        hipLaunchKernelGGL(gemm_tn_bf16_kernel<true>, dim3(grid), dim3(kThreads16), 0, stream, C, a, b, M, N, K, lda,
-                           ldb, ldc, alpha, ti, dp, sk, plan.parts, ws);
-    else
-        hipLaunchKernelGGL(gemm_tn_bf16_kernel<false>, dim3(grid), dim3(kThreads16), 0, stream, C, a, b, M, N, K, lda,
-                           ldb, ldc, alpha, ti, dp, sk, plan.parts, ws);
+    auto* kernel = sym ? (plan.staged ? gemm_tn_bf16_kernel<true, true> : gemm_tn_bf16_kernel<true, false>)
+                       : (plan.staged ? gemm_tn_bf16_kernel<false, true> : gemm_tn_bf16_kernel<false, false>);
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(kThreads16), 0, stream, C, a, b, M, N, K, lda, ldb, ldc, alpha, ti, dp,
+                       sk, plan.parts, ws);
     QSRT_HIP_TRY(hipGetLastError());
     if (plan.sk) {
         if (sym)
@@ -780,9 +833,31 @@ int qsrt_gemm_tn_ws(float* C, const void* A, const void* B, const void* B2, int6
     return qsrt::kOk;
 }
 
+}  // namespace
+
+extern "C" {
+
+size_t qsrt_gemm_tn_workspace_bytes(const float* C, const void* A, const void* B, int64_t M, int64_t N, int64_t K,
+                                    int64_t lda, int64_t ldb, int64_t ldc, int dtype) {
+    if (M <= 0 || N <= 0 || K <= 0) return 0;
+    if (dtype == 0 && f32_symmetric(C, A, B, nullptr, M, N, lda, ldb, ldc)) {
+        const int64_t tiles = f32_sym_tiles(M);
+        return gram_f32_workspace(tiles, gram_f32_parts(tiles, K, device_cus()));
+    }
+    if (dtype != 1) return 0;
+    const bool sym = bf16_symmetric(C, A, B, M, N, lda, ldb, ldc);
+    return bf16_plan(bf16_tiles(sym, M, N), (K + kBK16 - 1) / kBK16, device_cus()).workspace_bytes();
+}
+
+int qsrt_gemm_tn_ws(float* C, const void* A, const void* B, const void* B2, int64_t M, int64_t N, int64_t K,
+                    int64_t lda, int64_t ldb, int64_t ldc, float alpha, int dtype, void* workspace,
+                    size_t workspace_bytes, void* stream_handle) {
+    return gemm_tn(C, A, B, B2, M, N, K, lda, ldb, ldc, alpha, dtype, true, workspace, workspace_bytes, stream_handle);
+}
+
 int qsrt_gemm_tn(float* C, const void* A, const void* B, const void* B2, int64_t M, int64_t N, int64_t K,
                  int64_t lda, int64_t ldb, int64_t ldc, float alpha, int dtype, void* stream_handle) {
-    return qsrt_gemm_tn_ws(C, A, B, B2, M, N, K, lda, ldb, ldc, alpha, dtype, nullptr, 0, stream_handle);
+    return gemm_tn(C, A, B, B2, M, N, K, lda, ldb, ldc, alpha, dtype, false, nullptr, 0, stream_handle);
 }
 
 }  // extern "C"

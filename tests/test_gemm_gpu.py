@@ -234,6 +234,45 @@ def test_bf16_split_last_round(K, M, N, sym):
     assert int(moved.sum()) <= tiles % cus
 
 
+@pytest.mark.parametrize("K,M,N,sym", [(65, 4700, 4801, False), (128, 4700, 4801, False), (171, 7003, 7003, True),
+                                       (600, 7168, 7168, True), (1024, 7100, 7100, True)])
+def test_bf16_few_rows_behind_a_whole_round(K, M, N, sym):
+    """Few rows and more tiles than compute units: no partials, each stage of
+    64 rows summed by itself.  Products of bf16 are exact, so an element errs
+    by at most the additions it passes (64 in its stage, one per stage, alpha
+    and C), 2^-23 each of the sum of magnitudes if the matrix cores truncate;
+    shorter sums also err less (2-norm) than the plain kernel's."""
+
+    print(f"[gemm] bf16 few rows K{K} M{M} N{N} sym={sym}", file=sys.stderr, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(K + M + N)
+    ld = -(-max(M, N) // 8) * 8
+    A = torch.randn(K, ld, device="cuda", generator=g).bfloat16()[:, :M]
+    B = A if sym else torch.randn(K, ld, device="cuda", generator=g).bfloat16()[:, :N]
+    C0 = torch.randn(M, ld, device="cuda", generator=g)
+    if sym:
+        C0[:, :M] = C0[:, :M] + C0[:, :M].T.clone()
+    lib = _native.lib()
+    assert lib.qsrt_gemm_tn_workspace_bytes(C0.data_ptr(), A.data_ptr(), B.data_ptr(), M, N, K, A.stride(0),
+                                            B.stride(0), C0.stride(0), 1) == 0
+    none = torch.empty(0, dtype=torch.uint8, device="cuda")
+    staged, again, whole = C0.clone(), C0.clone(), C0.clone()
+    _bf16_call(staged[:, :N], A, B, 0.5, none)
+    _bf16_call(again[:, :N], A, B, 0.5, none)
+    _bf16_call(whole[:, :N], A, B, 0.5)
+    torch.cuda.synchronize()
+    assert torch.equal(staged, again)
+    assert torch.equal(staged[:, N:], C0[:, N:])  # nothing written past the columns
+    ref = C0[:, :N].double() + 0.5 * (A.double().T @ B.double())
+    size = C0[:, :N].abs().double() + 0.5 * (A.abs().double().T @ B.abs().double())
+    err = (staged[:, :N].double() - ref).abs()
+    assert (err <= (64 + -(-K // 64) + 2) * 2.0**-23 * size).all()
+    if K >= 128:  # below, one product is all that the second stage adds: no sum is shorter
+        assert not torch.equal(staged, whole)
+        assert err.norm() < (whole[:, :N].double() - ref).norm()
+    if sym:
+        assert torch.equal(staged[:, :N], staged[:, :N].T)
+
+
 def test_gemm_rejects_bad_arguments():
     A = torch.randn(4, 4).cuda()
     with pytest.raises(ValueError):
