@@ -236,10 +236,11 @@ int qsrt_decode_noalloc(const qsrt_decode_job *jobs, int n_jobs, int K, const ui
  * One uniform-rate matrix with the payload's own FP16 scales:
  *   words i16 [rows / 16, cols / 16, 16 K], suh f16 [rows], svh f16 [cols]
  *   -> out[r * out_ld + c] (bf16 or f32 as out_dtype says).
- * The result of qsrt_decode on the FP8 matrix-core path (a LUT with
- * |label| <= 6) with row_scale = suh / 128 and col_scale = svh, in one launch:
- * the job rides in the kernel's arguments and the scales are widened where
- * they are read, so nothing is uploaded or converted first and no workspace is
+ * The result of qsrt_decode with row_scale = suh / 128, col_scale = svh and the
+ * exact_fp8 that the table's labels call for: the kernels of both paths are
+ * launched and each decides from the table whether it is the one to run.  The
+ * job rides in the kernels' arguments and the scales are widened where they
+ * are read, so nothing is uploaded or converted first and no workspace is
  * needed.  rows and cols multiples of 128, K 2..4, words, out and lut_e4m3
  * 16-byte aligned, out_ld >= cols and a multiple of 8.  Replaces
  * decode_exl3_weight (qsrt/exl3_reference.py:280-302).

@@ -53,7 +53,6 @@ namespace {
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef const __attribute__((address_space(1))) uint32_t* gu32;
-typedef const __attribute__((address_space(1))) float* gf32;
 typedef const __attribute__((address_space(1))) f32x4* gf4;
 
 constexpr int kWaves = 8;
@@ -114,7 +113,6 @@ struct BlockCtxOf {
     char* out;             // element (128 br, 128 bc)
     int64_t ld;
 };
-using BlockCtx = BlockCtxOf<float>;
 
 template <typename Scale = float>
 __device__ __forceinline__ BlockCtxOf<Scale> block_ctx(const Job* jobs, const Cursor& cu, int out_size) {
@@ -159,10 +157,49 @@ __device__ __forceinline__ uint32_t residual_pair(uint32_t hi, float e0, float e
     return __builtin_bit_cast(uint32_t, lo);
 }
 
-template <int K, typename OutT>
+// Where a launch's jobs are: a table in device memory with FP32 scales (row
+// scales already divided by 128), or one job in the kernel's own argument with
+// the payload's FP16 scales, which needs no upload and no conversion launch.
+struct JobTable {
+    static constexpr bool kPicksKernel = false;  // the caller has chosen between the FP8 and the FP32 kernel
+    typedef float Scale;
+    const Job* table;
+    __device__ const Job* jobs() const { return table; }
+    __device__ static float row_scale(float v) { return v; }
+};
+struct OneJob {
+    // Both kernels are launched, and each looks at its table: the one that it is not for ends.  The host would have to
+    // wait for the table's bound on every call, and nothing of an earlier call says what the table holds now. 7168 x 2048
+    // at K3: 23 us a pass for both, 18 without the second launch and the two looks at the table, 82 with the host's.
+    static constexpr bool kPicksKernel = true;
+    typedef _Float16 Scale;
+    Job job;
+    __device__ const Job* jobs() const { return &job; }
+    __device__ static float row_scale(_Float16 v) { return static_cast<float>(v) * 0.0078125f; }
+};
+
+// Whether any thread of the workgroup passes true; `word` is LDS that is free before and after (__syncthreads_or would
+// take its own, and with it the FP32 kernel's second workgroup per CU).
+__device__ __forceinline__ bool any_thread(bool mine, uint32_t* word) {
+    if (threadIdx.x == 0) *word = 0;
+    __syncthreads();
+    if (mine) *word = 1;
+    __syncthreads();
+    const bool any = *word != 0;
+    __syncthreads();
+    return any;
+}
+
+// Whether a dword of the table holds a label that the FP8 products are not exact for (beyond 6.0, 0x4C, or NaN).
+__device__ __forceinline__ uint32_t large_labels(uint32_t v) { return ((v & 0x7F7F7F7Fu) + 0x33333333u) & 0x80808080u; }
+
+template <int K, typename OutT, typename Source>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4)))
-void decode_fp32_kernel(const Job* __restrict__ jobs, int n_jobs, int64_t total_blocks, const uint8_t* __restrict__ lut) {
+void decode_fp32_kernel(const Source source, int n_jobs, int64_t total_blocks, const uint8_t* __restrict__ lut) {
     static_assert(sizeof(OutT) == 2 || sizeof(OutT) == 4, "bf16 or f32 output");
+    typedef typename Source::Scale Scale;
+    typedef const __attribute__((address_space(1))) Scale* gscale;
+    const Job* const jobs = source.jobs();
     __shared__ __attribute__((aligned(16))) uint8_t lut_s[65536];
     // Label area, 2 KB per wave.  During B1: labels of tile-column a', lane l,
     // half h (tile-rows 4h..4h+3) at ((a' * 2 + h) * 64 + l) * 16.  Wave w's
@@ -175,6 +212,14 @@ void decode_fp32_kernel(const Job* __restrict__ jobs, int n_jobs, int64_t total_
     const int64_t end = total_blocks * (blockIdx.x + 1) / gridDim.x;
     if (begin >= end) return;
 
+    if constexpr (Source::kPicksKernel) {
+        uint32_t large = 0;
+        for (int i = threadIdx.x; i < 65536 / 16; i += kThreads) {
+            const uint4 v = reinterpret_cast<const uint4*>(lut)[i];
+            large |= large_labels(v.x) | large_labels(v.y) | large_labels(v.z) | large_labels(v.w);
+        }
+        if (!any_thread(large != 0, reinterpret_cast<uint32_t*>(labels))) return;  // decode_block_wave_kernel's table
+    }
     for (int i = threadIdx.x; i < 65536 / 16; i += kThreads)
         reinterpret_cast<uint4*>(lut_s)[i] = reinterpret_cast<const uint4*>(lut)[i];
 
@@ -210,12 +255,12 @@ void decode_fp32_kernel(const Job* __restrict__ jobs, int n_jobs, int64_t total_
     const uint32_t* wstage = reinterpret_cast<const uint32_t*>(slice);
 
     Cursor cu = cursor_at(jobs, n_jobs, begin);
-    BlockCtx ctx = block_ctx(jobs, cu, sizeof(OutT));
+    BlockCtxOf<Scale> ctx = block_ctx<Scale>(jobs, cu, sizeof(OutT));
     u32x4 words = fetch_words<K>(ctx, w, lane);
-    float su = ((gf32)ctx.su)[16 * w + c];
+    float su = Source::row_scale(((gscale)ctx.su)[16 * w + c]);
     float sv[8];
 #pragma unroll
-    for (int a = 0; a < 8; ++a) sv[a] = ((gf32)ctx.sv)[16 * a + c];
+    for (int a = 0; a < 8; ++a) sv[a] = static_cast<float>(((gscale)ctx.sv)[16 * a + c]);
     __syncthreads();
 
     for (int64_t blk = begin; blk < end; ++blk) {
@@ -239,15 +284,15 @@ void decode_fp32_kernel(const Job* __restrict__ jobs, int n_jobs, int64_t total_
 #pragma unroll
         for (int a = 0; a < 8; ++a) svf[a] = sv[a];
         const float su_cur = su;
-        const BlockCtx cur = ctx;
+        const BlockCtxOf<Scale> cur = ctx;
         // ---- prefetch the next block (before this block's stores)
         if (blk + 1 < end) {
             cursor_next(jobs, cu);
-            ctx = block_ctx(jobs, cu, sizeof(OutT));
+            ctx = block_ctx<Scale>(jobs, cu, sizeof(OutT));
             words = fetch_words<K>(ctx, w, lane);
-            su = ((gf32)ctx.su)[16 * w + c];
+            su = Source::row_scale(((gscale)ctx.su)[16 * w + c]);
 #pragma unroll
-            for (int a = 0; a < 8; ++a) sv[a] = ((gf32)ctx.sv)[16 * a + c];
+            for (int a = 0; a < 8; ++a) sv[a] = static_cast<float>(((gscale)ctx.sv)[16 * a + c]);
         }
         __syncthreads();
 
@@ -369,22 +414,6 @@ __device__ __forceinline__ BlockCtxOf<Scale> uniform_ctx(BlockCtxOf<Scale> x) {
     return x;
 }
 
-// Where a launch's jobs are: a table in device memory with FP32 scales (row
-// scales already divided by 128), or one job in the kernel's own argument with
-// the payload's FP16 scales, which needs no upload and no conversion launch.
-struct JobTable {
-    typedef float Scale;
-    const Job* table;
-    __device__ const Job* jobs() const { return table; }
-    __device__ static float row_scale(float v) { return v; }
-};
-struct OneJob {
-    typedef _Float16 Scale;
-    Job job;
-    __device__ const Job* jobs() const { return &job; }
-    __device__ static float row_scale(_Float16 v) { return static_cast<float>(v) * 0.0078125f; }
-};
-
 template <int K, typename OutT, typename Source>
 __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(3, 3)))
 void decode_block_wave_kernel(const Source source, int n_jobs, int64_t total_blocks,
@@ -428,7 +457,15 @@ void decode_block_wave_kernel(const Source source, int n_jobs, int64_t total_blo
         __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(lut + 1024 * i + 16 * lane),
                                          (__attribute__((address_space(3))) void*)(lut_s + 1024 * i), 16, 0, 0);
     __builtin_amdgcn_s_waitcnt(0);  // vmcnt(0): the builtin's writes to LDS are not ordered by the barrier alone
-    __syncthreads();  // the kernel's only barrier
+    __syncthreads();  // the kernel's only barrier, but for the check of a table that no caller has looked at
+    if constexpr (Source::kPicksKernel) {
+        uint32_t large = 0;
+        for (int i = threadIdx.x; i < 65536 / 16; i += 64 * waves) {
+            const uint4 v = reinterpret_cast<const uint4*>(lut_s)[i];
+            large |= large_labels(v.x) | large_labels(v.y) | large_labels(v.z) | large_labels(v.w);
+        }
+        if (any_thread(large != 0, reinterpret_cast<uint32_t*>(slices))) return;  // decode_fp32_kernel's table
+    }
     if (begin >= end) return;
 
     const int g = lane >> 4;
@@ -639,20 +676,25 @@ void launch_block_wave_k(const Source& source, int n_jobs, int64_t total, const 
                            total, lut);
 }
 
+template <int K, typename Source>
+void launch_fp32_k(const Source& source, int n_jobs, int64_t total, const uint8_t* lut, int out_dtype, int cus,
+                   hipStream_t stream) {
+    const unsigned grid = static_cast<unsigned>(std::min<int64_t>(2 * static_cast<int64_t>(cus), total));  // 2 per CU
+    if (out_dtype == 0)
+        hipLaunchKernelGGL((decode_fp32_kernel<K, __bf16, Source>), dim3(grid), dim3(kThreads), 0, stream, source,
+                           n_jobs, total, lut);
+    else
+        hipLaunchKernelGGL((decode_fp32_kernel<K, float, Source>), dim3(grid), dim3(kThreads), 0, stream, source, n_jobs,
+                           total, lut);
+}
+
 template <int K, bool FP8>
 void launch(const Job* jobs, int n_jobs, int64_t total, const uint8_t* lut, int out_dtype, int cus,
             hipStream_t stream) {
-    if constexpr (FP8) {
+    if constexpr (FP8)
         launch_block_wave_k<K>(JobTable{jobs}, n_jobs, total, lut, out_dtype, cus, stream);
-    } else {
-        const unsigned grid = static_cast<unsigned>(std::min<int64_t>(2 * static_cast<int64_t>(cus), total));  // 2 per CU
-        if (out_dtype == 0)
-            hipLaunchKernelGGL((decode_fp32_kernel<K, __bf16>), dim3(grid), dim3(kThreads), 0, stream, jobs, n_jobs,
-                               total, lut);
-        else
-            hipLaunchKernelGGL((decode_fp32_kernel<K, float>), dim3(grid), dim3(kThreads), 0, stream, jobs, n_jobs,
-                               total, lut);
-    }
+    else
+        launch_fp32_k<K>(JobTable{jobs}, n_jobs, total, lut, out_dtype, cus, stream);
 }
 
 // Job-table upload by kernel argument: the host validates and converts up to
@@ -869,9 +911,17 @@ extern "C" int qsrt_decode_matrix_f16(const int16_t* words, int64_t rows, int64_
     if (const int rc = qsrt::current_cu_count(&cus)) return rc;
     const OneJob source{device_job(s, 0)};
     const int64_t total = (rows / 128) * (cols / 128);
-    auto* launch = K == 2 ? launch_block_wave_k<2, OneJob> : K == 3 ? launch_block_wave_k<3, OneJob>
-                                                                    : launch_block_wave_k<4, OneJob>;
-    launch(source, 1, total, lut_e4m3, out_dtype, cus, static_cast<hipStream_t>(stream_handle));
+    hipStream_t stream = static_cast<hipStream_t>(stream_handle);
+    const auto both = [&](auto* wave, auto* fp32) {
+        wave(source, 1, total, lut_e4m3, out_dtype, cus, stream);
+        fp32(source, 1, total, lut_e4m3, out_dtype, cus, stream);
+    };
+    if (K == 2)
+        both(launch_block_wave_k<2, OneJob>, launch_fp32_k<2, OneJob>);
+    else if (K == 3)
+        both(launch_block_wave_k<3, OneJob>, launch_fp32_k<3, OneJob>);
+    else
+        both(launch_block_wave_k<4, OneJob>, launch_fp32_k<4, OneJob>);
     QSRT_HIP_TRY(hipGetLastError());
     return qsrt::kOk;
 }

@@ -250,3 +250,27 @@ def test_payload_scales_equal_converted_scales(bits, shape):
         got = D.decode_words(words, suh, svh, bits, lut, out_dtype=dtype, out=out[:, :n])
         assert torch.equal(got, want)
         assert not out[:, n:].any()
+
+
+@pytest.mark.parametrize("at,byte", ((0, 0x4C), (65535, 0xCC), (0, 0x4D), (65535, 0xCD), (40000, 0x7F), (4097, 0xFE)))
+@pytest.mark.parametrize("bits,shape", ((2, (128, 128)), (3, (384, 128 * 171)), (4, (256, 128 * 129))))
+def test_payload_scales_follow_the_table_as_it_is(bits, shape, at, byte):
+    """One label at or past the FP8 path's bound (6.0 is 0x4C), or NaN, written into a table already decoded with, behind
+    the tensor's version counter: the same kernel, hence the same bits, as the route that looks at the table from the
+    host; 1, 513 and 258 blocks."""
+
+    k, n = shape
+    print(f"[decode] K{bits} {k} x {n}, label {byte:#x} at {at}", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(bits * 31 + k + n)
+    words = torch.randint(-32768, 32768, (k // 16, n // 16, 16 * bits), generator=gen, device="cuda",
+                          dtype=torch.int32).to(torch.int16)
+    suh = (torch.rand(k, generator=gen, device="cuda") + 0.5).half()
+    svh = torch.randn(n, generator=gen, device="cuda").half()
+    lut = sqg_xor_cheb_t12_bytes(bits).cuda()
+    D.decode_words(words, suh, svh, bits, lut)
+    lut.data[at] = byte
+    for dtype in (torch.bfloat16, torch.float32):
+        got = D.decode_words(words, suh, svh, bits, lut, out_dtype=dtype)
+        want = D.decode_words(words, suh.float(), svh.float(), bits, lut.clone(), out_dtype=dtype)
+        assert torch.equal(got.isnan(), want.isnan())
+        assert torch.equal(got.nan_to_num(), want.nan_to_num())
