@@ -55,9 +55,9 @@ FP32_UNPACKED_PEAK_TFLOPS = 78.6  # 256 CUs x 64 FP32 FMA lanes x 2 flops x 2.4 
 HBM_PEAK_GBPS = 8000.0
 MFMA_PEAK_TFLOPS = {"bf16": 2500.0, "f32": 157.3, "f64": 78.6}
 # HBM bytes per tile of the Viterbi kernel by rate (FETCH_SIZE x 2.00 + WRITE_SIZE x 1.00 per dispatch, calibrated
-# on a 4 GiB device copy; K3/K4 over every dispatch of a 20-expert layer step, K2 from the microbench;
-# profiles/layer_encode_config5.md): mostly the traceback decision stream.
-VITERBI_HBM_BYTES_PER_TILE = {2: 1.631e6, 3: 1.633e6, 4: 0.816e6}
+# on a 4 GiB device copy; 8,192-tile dispatches, profiles/viterbi_tiles_kernel_microbench.md): mostly the cost
+# checkpoints.
+VITERBI_HBM_BYTES_PER_TILE = {2: 7.829e6, 3: 4.727e6, 4: 3.928e6}
 # Same counters for the decode launches: 1.03 x their algorithmic bytes (profiles/decode_kernel_layer.md).
 DECODE_TRAFFIC_OVER_ALGORITHMIC = 1.032
 # Same counters at the bench's GEMM and Hadamard shapes (profiles/gemm_tn_kernels_expert_shapes.md,
@@ -1178,8 +1178,8 @@ def headline(lay: dict, warmup: int) -> dict:
             "frac": round(achieved / FP32_PEAK_TFLOPS, 4),
             "traffic": round(sum(VITERBI_HBM_BYTES_PER_TILE[int(k[1:])] * d["tiles"] for k, d in vit["by_rate"].items())
                              / max(vit["launches"], 1)),
-            "traffic_note": TRAFFIC_NOTE.format("profiles/layer_encode_config5.md"),
-            "kernel": "viterbi_tiles_kernel",
+            "traffic_note": TRAFFIC_NOTE.format("profiles/viterbi_tiles_kernel_microbench.md"),
+            "kernel": "viterbi_cone_kernel",
             "algorithmic": f"{FLOPS_PER_EDGE} FP32 flops/edge x {int(EDGES_PER_WEIGHT)} edges/weight x 256 weights/tile "
                            f"x {mean_tiles:.1f} tiles/launch (mean over {vit['launches']} launches in the timed region)",
             "mean_launch_ms": round(mean_launch_ms, 4),
