@@ -170,7 +170,7 @@ struct JobTable {
 struct OneJob {
     // Both kernels are launched, and each looks at its table: the one that it is not for ends.  The host would have to
     // wait for the table's bound on every call, and nothing of an earlier call says what the table holds now. 7168 x 2048
-    // at K3: 23 us a pass for both, 18 without the second launch and the two looks at the table, 82 with the host's.
+    // at K3: 22 us a pass for both, 18 without the second launch and the two looks at the table, 82 with the host's.
     static constexpr bool kPicksKernel = true;
     typedef _Float16 Scale;
     Job job;
@@ -214,8 +214,9 @@ void decode_fp32_kernel(const Source source, int n_jobs, int64_t total_blocks, c
 
     if constexpr (Source::kPicksKernel) {
         uint32_t large = 0;
-        for (int i = threadIdx.x; i < 65536 / 16; i += kThreads) {
-            const uint4 v = reinterpret_cast<const uint4*>(lut)[i];
+#pragma unroll
+        for (int q = 0; q < 65536 / 16 / kThreads; ++q) {  // every load in flight: the launch is nothing but this look
+            const uint4 v = reinterpret_cast<const uint4*>(lut)[threadIdx.x + q * kThreads];
             large |= large_labels(v.x) | large_labels(v.y) | large_labels(v.z) | large_labels(v.w);
         }
         if (!any_thread(large != 0, reinterpret_cast<uint32_t*>(labels))) return;  // decode_block_wave_kernel's table
@@ -460,6 +461,7 @@ void decode_block_wave_kernel(const Source source, int n_jobs, int64_t total_blo
     __syncthreads();  // the kernel's only barrier, but for the check of a table that no caller has looked at
     if constexpr (Source::kPicksKernel) {
         uint32_t large = 0;
+#pragma unroll 4
         for (int i = threadIdx.x; i < 65536 / 16; i += 64 * waves) {
             const uint4 v = reinterpret_cast<const uint4*>(lut_s)[i];
             large |= large_labels(v.x) | large_labels(v.y) | large_labels(v.z) | large_labels(v.w);
