@@ -83,7 +83,8 @@ struct Cursor {
 };
 
 // Cursor of block `blk`: binary search over the jobs' block prefix.
-__device__ __forceinline__ Cursor cursor_at(const Job* jobs, int n_jobs, int64_t blk) {
+template <typename Jobs>
+__device__ __forceinline__ Cursor cursor_at(Jobs jobs, int n_jobs, int64_t blk) {
     int lo = 0, hi = n_jobs - 1;  // jobs[lo].first_block <= blk < jobs[hi + 1].first_block
     while (lo < hi) {
         const int mid = (lo + hi + 1) >> 1;
@@ -94,7 +95,8 @@ __device__ __forceinline__ Cursor cursor_at(const Job* jobs, int n_jobs, int64_t
     return Cursor{lo, br, static_cast<int>(local - static_cast<int64_t>(br) * jobs[lo].nbc)};
 }
 
-__device__ __forceinline__ void cursor_next(const Job* jobs, Cursor& cu) {
+template <typename Jobs>
+__device__ __forceinline__ void cursor_next(Jobs jobs, Cursor& cu) {
     if (++cu.bc == jobs[cu.j].nbc) {
         cu.bc = 0;
         if (++cu.br == jobs[cu.j].nbr) {
@@ -114,9 +116,9 @@ struct BlockCtxOf {
     int64_t ld;
 };
 
-template <typename Scale = float>
-__device__ __forceinline__ BlockCtxOf<Scale> block_ctx(const Job* jobs, const Cursor& cu, int out_size) {
-    const Job& J = jobs[cu.j];
+template <typename Scale, typename Jobs>
+__device__ __forceinline__ BlockCtxOf<Scale> block_ctx(Jobs jobs, const Cursor& cu, int out_size) {
+    const auto& J = jobs[cu.j];
     BlockCtxOf<Scale> x;
     x.words = J.words + cu.br * J.block_row_stride + cu.bc * J.block_col_stride;
     x.trs = J.tile_row_stride;
@@ -164,7 +166,10 @@ struct JobTable {
     static constexpr bool kPicksKernel = false;  // the caller has chosen between the FP8 and the FP32 kernel
     typedef float Scale;
     const Job* table;
-    __device__ const Job* jobs() const { return table; }
+    // Constant for the kernel, so that a wave reads its jobs by scalar loads whatever it has stored in between (8192
+    // blocks of the FP32 kernel at K3: 703 us, by vector loads 729).
+    typedef const __attribute__((address_space(4))) Job* ConstJob;
+    __device__ ConstJob jobs() const { return (ConstJob)table; }
     __device__ static float row_scale(float v) { return v; }
 };
 struct OneJob {
@@ -199,7 +204,7 @@ void decode_fp32_kernel(const Source source, int n_jobs, int64_t total_blocks, c
     static_assert(sizeof(OutT) == 2 || sizeof(OutT) == 4, "bf16 or f32 output");
     typedef typename Source::Scale Scale;
     typedef const __attribute__((address_space(1))) Scale* gscale;
-    const Job* const jobs = source.jobs();
+    const auto jobs = source.jobs();
     __shared__ __attribute__((aligned(16))) uint8_t lut_s[65536];
     // Label area, 2 KB per wave.  During B1: labels of tile-column a', lane l,
     // half h (tile-rows 4h..4h+3) at ((a' * 2 + h) * 64 + l) * 16.  Wave w's
@@ -387,6 +392,7 @@ void decode_fp32_kernel(const Source source, int n_jobs, int64_t total_blocks, c
 // every pipe busy at once.
 constexpr int kBlockWaves = 12;  // one workgroup of at most 12 waves per CU (3 per SIMD)
 constexpr int kBlockThreads = 64 * kBlockWaves;
+constexpr int kCopyWaves = 4;    // waves of a workgroup at the least: the table's copy
 constexpr int kSliceBytes = 2048;  // half an output tile-row of bf16 (16 rows x 128 B); a tile-column's words
 constexpr int kScaleBytes = 1024;  // a block's su (128 f32) and fp16-paired sv (128 x 2 fp16)
 
@@ -415,6 +421,24 @@ __device__ __forceinline__ BlockCtxOf<Scale> uniform_ctx(BlockCtxOf<Scale> x) {
     return x;
 }
 
+// Find block `begin` and request its words and scales.
+template <int K, typename Source, typename Scale = typename Source::Scale>
+__device__ __forceinline__ void first_block(const Source& source, int n_jobs, int64_t begin, int out_size, Cursor& cu,
+                                            BlockCtxOf<Scale>& ctx, u32x4 (&words)[8], float (&su_n)[8],
+                                            float (&sv_n)[8]) {
+    typedef const __attribute__((address_space(1))) Scale* gscale;
+    const int lane = threadIdx.x & 63, c = lane & 15;
+    cu = cursor_at(source.jobs(), n_jobs, begin);
+    ctx = uniform_ctx(block_ctx<Scale>(source.jobs(), cu, out_size));
+#pragma unroll
+    for (int col = 0; col < 8; ++col) words[col] = fetch_words<K>(ctx, col, lane);
+#pragma unroll
+    for (int a = 0; a < 8; ++a) {
+        su_n[a] = Source::row_scale(((gscale)ctx.su)[16 * a + c]);
+        sv_n[a] = static_cast<float>(((gscale)ctx.sv)[16 * a + c]);
+    }
+}
+
 template <int K, typename OutT, typename Source>
 __global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(3, 3)))
 void decode_block_wave_kernel(const Source source, int n_jobs, int64_t total_blocks,
@@ -426,7 +450,7 @@ void decode_block_wave_kernel(const Source source, int n_jobs, int64_t total_blo
     __shared__ __attribute__((aligned(16))) uint8_t slices[kBlockWaves * kSliceBytes];
     __shared__ __attribute__((aligned(16))) uint8_t scales[kBlockWaves * kScaleBytes];
 
-    const Job* const jobs = source.jobs();
+    const auto jobs = source.jobs();
     const int waves = static_cast<int>(blockDim.x) >> 6;
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -435,22 +459,17 @@ void decode_block_wave_kernel(const Source source, int n_jobs, int64_t total_blo
     const int64_t begin = sgpr64(total_blocks * gw / nw);
     const int64_t end = sgpr64(total_blocks * (gw + 1) / nw);
 
-    // The first block's words and scales are requested ahead of the table: a wave of a small launch decodes one block.
     const int c = lane & 15;
     Cursor cu{};
     BlockCtxOf<Scale> ctx{};
     u32x4 words[8];
     float su_n[8], sv_n[8];
-    if (begin < end) {
-        cu = cursor_at(jobs, n_jobs, begin);
-        ctx = uniform_ctx(block_ctx<Scale>(jobs, cu, sizeof(OutT)));
-#pragma unroll
-        for (int col = 0; col < 8; ++col) words[col] = fetch_words<K>(ctx, col, lane);
-#pragma unroll
-        for (int a = 0; a < 8; ++a) {
-            su_n[a] = Source::row_scale(((gscale)ctx.su)[16 * a + c]);
-            sv_n[a] = static_cast<float>(((gscale)ctx.sv)[16 * a + c]);
-        }
+    // One job: the first block's words and scales are requested ahead of the table, as a wave of a small launch decodes
+    // one block.  A job table's waves ask for theirs behind the barrier: each then starts when its own search of the
+    // jobs and its own loads are done, and not all twelve at once on the gathers (8192 blocks at K4 in one table: 89.5
+    // us with the words first, 86.0 this way).
+    if constexpr (Source::kPicksKernel) {
+        if (begin < end) first_block<K>(source, n_jobs, begin, sizeof(OutT), cu, ctx, words, su_n, sv_n);
     }
     // The table goes to LDS without passing through registers, every load in flight at once: copied 16 bytes per
     // thread and round trip, a workgroup of 4 waves spent 16 round trips on it, half of a one-block launch.
@@ -469,6 +488,7 @@ void decode_block_wave_kernel(const Source source, int n_jobs, int64_t total_blo
         if (any_thread(large != 0, reinterpret_cast<uint32_t*>(slices))) return;  // decode_fp32_kernel's table
     }
     if (begin >= end) return;
+    if constexpr (!Source::kPicksKernel) first_block<K>(source, n_jobs, begin, sizeof(OutT), cu, ctx, words, su_n, sv_n);
 
     const int g = lane >> 4;
     const int rho[4] = {2 * g, 2 * g + 1, 2 * g + 8, 2 * g + 9};
@@ -661,7 +681,11 @@ void decode_block_wave_kernel(const Source source, int n_jobs, int64_t total_blo
 // the other CUs idle (32.5 -> 18.9 us at K3 under the trace, the table copy
 // included).  Cutting such blocks further, into parts of their tile-rows on
 // twice the waves, was no faster (20.3 us): the label phase, which every part
-// repeats, is what a lone wave takes its time for.
+// repeats, is what a lone wave takes its time for.  Past one round of twelve
+// waves the even share is the better one too (a table of 3200 blocks at K3: 43.8
+// us on twelve waves a CU, 38.8 on seven; 5376: 54.8 and 52.3).  A workgroup
+// has four waves at least: those without a block copy the table and end (one
+// block: 13.9 us with one wave, 12.8 with four).
 template <int K, typename Source>
 void launch_block_wave_k(const Source& source, int n_jobs, int64_t total, const uint8_t* lut, int out_dtype, int cus,
                          hipStream_t stream) {
@@ -669,7 +693,7 @@ void launch_block_wave_k(const Source& source, int n_jobs, int64_t total, const 
     const int64_t rounds = (total + per_round - 1) / per_round;
     const int64_t waves = (total + rounds * cus - 1) / (rounds * cus);
     const unsigned grid = static_cast<unsigned>(std::min<int64_t>(cus, (total + waves - 1) / waves));
-    const dim3 block(static_cast<unsigned>(64 * waves));
+    const dim3 block(static_cast<unsigned>(64 * std::max<int64_t>(waves, kCopyWaves)));
     if (out_dtype == 0)
         hipLaunchKernelGGL((decode_block_wave_kernel<K, __bf16, Source>), dim3(grid), block, 0, stream, source, n_jobs,
                            total, lut);

@@ -274,3 +274,30 @@ def test_payload_scales_follow_the_table_as_it_is(bits, shape, at, byte):
         want = D.decode_words(words, suh.float(), svh.float(), bits, lut.clone(), out_dtype=dtype)
         assert torch.equal(got.isnan(), want.isnan())
         assert torch.equal(got.nan_to_num(), want.nan_to_num())
+
+
+@pytest.mark.parametrize("shape", ((1, 1), (1, 5), (2, 128), (1, 257), (3, 257), (25, 123)))
+def test_blocks_decode_alike_alone_and_together(shape):
+    """Workgroups whose waves outnumber their blocks (1, 5, 256 and 257 blocks; at 771 all four have one) and a second
+    round (3075): every 128 x 128 block is, bit for bit, what a call of its own makes of it, as a job table and as one
+    matrix.  A wave per block does the same arithmetic whatever it is launched with."""
+
+    rows, cols = shape
+    bits, k, n = 4, 128 * rows, 128 * cols
+    _say(f"[decode] {rows} x {cols} blocks alone and together")
+    gen = torch.Generator(device="cuda").manual_seed(k + n)
+    words = torch.randint(-32768, 32768, (k // 16, n // 16, 16 * bits), generator=gen, device="cuda",
+                          dtype=torch.int32).to(torch.int16)
+    suh = (torch.rand(k, generator=gen, device="cuda") + 0.5).half()
+    svh = torch.randn(n, generator=gen, device="cuda").half()
+    lut = sqg_xor_cheb_t12_bytes(bits).cuda()
+    want = torch.full((k, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+    for block in range(0, rows * cols, 1 + rows * cols // 300):
+        r, c = divmod(block, cols)
+        at = (slice(128 * r, 128 * r + 128), slice(128 * c, 128 * c + 128))
+        D.decode_words(words[8 * r:8 * r + 8, 8 * c:8 * c + 8], suh[at[0]], svh[at[1]], bits, lut, out=want[at])
+    seen = ~want.isnan()
+    for row_scale, col_scale in ((suh, svh), (suh.float(), svh.float())):
+        got = D.decode_words(words, row_scale, col_scale, bits, lut)
+        assert not got.isnan().any()
+        assert torch.equal(got[seen], want[seen])
