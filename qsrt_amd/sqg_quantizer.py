@@ -36,29 +36,30 @@ from .sqg_e4m3 import sqg_e4m3_bytes
 # kernel (qsrt_quantize_tiles_k2_kernel.cuh:45).
 K2_FAST_MAX_LABEL = 16.0
 
-_workspaces: dict[tuple[int, int], torch.Tensor] = {}
+# Bytes per workgroup of the traceback that records decisions, for the rates that have checkpoints instead.
+_RECORDED_BYTES = {2: 2 << 20, 3: 2 << 20, 4: 1 << 20}
 
 
-def _workspace(device: torch.device, bits: int, n_tiles: int) -> torch.Tensor:
-    """Traceback workspace of the current stream on ``device``.  Each stream
-    has its own buffer (sized once for the widest grid), so launches queued
-    on different streams never share decision rows; launches on one stream
-    are ordered and reuse it."""
+def _workspace(device: torch.device, bits: int, workgroups: int) -> torch.Tensor:
+    """Traceback workspace of one launch on the current stream of ``device``,
+    for ``workgroups`` of them (or one per CU, if that is fewer), from torch's
+    stream-ordered allocator: launches queued on different streams never share
+    it, and nothing is held between calls.  Where the cost checkpoints do not
+    fit the device, a buffer for the recorded decisions (a quarter of the size
+    at K2 and K4, the same results) selects that traceback."""
 
-    need = int(_native.lib().qsrt_viterbi_workspace_bytes(bits, n_tiles))
+    need = int(_native.lib().qsrt_viterbi_workspace_bytes(bits, workgroups))
     if need == 0:
         raise _native.NativeError(
             "qsrt_viterbi_workspace_bytes failed: " + _native.lib().qsrt_last_error().decode()
         )
-    index = device.index if device.index is not None else torch.cuda.current_device()
-    key = (index, torch.cuda.current_stream(device).cuda_stream)
-    ws = _workspaces.get(key)
-    if ws is None or ws.numel() < need:
-        # Size for the widest grid (one workgroup per CU) once.
-        full = max(int(_native.lib().qsrt_viterbi_workspace_bytes(b, 1 << 30)) for b in range(1, 7))
-        ws = torch.empty(max(need, full), dtype=torch.uint8, device=device)
-        _workspaces[key] = ws
-    return ws
+    try:
+        return torch.empty(need, dtype=torch.uint8, device=device)
+    except torch.OutOfMemoryError:
+        if bits not in _RECORDED_BYTES:
+            raise
+        grid = min(workgroups, torch.cuda.get_device_properties(device).multi_processor_count)
+        return torch.empty(grid * _RECORDED_BYTES[bits], dtype=torch.uint8, device=device)
 
 
 def _lut_abs_max(lut: torch.Tensor) -> float:
@@ -137,8 +138,8 @@ def viterbi_tiles(
     n = tiles.shape[0]
     if n == 0:
         return recon, states
-    ws = _workspace(tiles.device, bits, n)
     with torch.cuda.device(tiles.device):
+        ws = _workspace(tiles.device, bits, min(n, max_workgroups) if max_workgroups > 0 else n)
         rc = _native.lib().qsrt_viterbi_tiles_ex(
             tiles.data_ptr(), recon.data_ptr(), states.data_ptr(), n, int(bits), int(tailbite_context),
             lut.data_ptr(), int(lag), int(max_workgroups), ws.data_ptr(), ws.numel(),

@@ -65,3 +65,47 @@ def test_checkpoints_equal_recorded_decisions(bits):
     differ = (states != s2).any(dim=1).nonzero().flatten().tolist()
     assert not differ, f"tiles {differ[:8]} differ"
     assert torch.equal(recon, r2)
+
+
+@pytest.mark.parametrize("bits,n,cap", [(4, 1, 0), (2, 3, 0), (3, 300, 10), (4, 300, 0)])
+def test_workspace_is_sized_by_the_launch_and_given_back(bits, n, cap):
+    """A call takes what its own rate and grid use, and holds none of it afterwards."""
+
+    print(f"[viterbi] K{bits}: {n} tiles on at most {cap} workgroups, memory", file=sys.stderr, flush=True)
+    tiles = torch.randn((n, 256), device="cuda")
+    lut = sqg_xor_cheb_t12_bytes(bits).cuda()
+    with torch.cuda.stream(torch.cuda.Stream()):
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        out = viterbi_tiles(tiles, lut, bits, max_workgroups=cap)
+        torch.cuda.synchronize()
+        peak = torch.cuda.max_memory_allocated() - before
+        kept = torch.cuda.memory_allocated() - before
+    results = 2 * 512 + sum(t.numel() * t.element_size() for t in out)  # blocks of the allocator are whole 512 bytes
+    assert kept <= results
+    # and a large one is not cut where 1 MiB or less would be left over
+    assert peak <= results + (1 << 20) + _native.lib().qsrt_viterbi_workspace_bytes(bits, cap or n)
+
+
+@pytest.mark.parametrize("bits", (2, 3, 4))
+def test_checkpoints_that_do_not_fit_give_way_to_recorded_decisions(bits):
+    n = 300
+    print(f"[viterbi] K{bits}: {n} tiles, memory for the recorded decisions only", file=sys.stderr, flush=True)
+    tiles = torch.randn((n, 256), device="cuda")
+    lut = sqg_xor_cheb_t12_bytes(bits).cuda()
+    recon, states = viterbi_tiles(tiles, lut, bits)
+    recorded = torch.cuda.get_device_properties(0).multi_processor_count * (1 << 20 if bits == 4 else 2 << 20)
+    assert recorded < _native.lib().qsrt_viterbi_workspace_bytes(bits, n)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    # the allocator's own limit, far below the card's memory; 64 MiB for the results and whole segments
+    limit = torch.cuda.memory_reserved() + recorded + (64 << 20)
+    torch.cuda.set_per_process_memory_fraction(limit / torch.cuda.get_device_properties(0).total_memory)
+    try:
+        with torch.cuda.stream(torch.cuda.Stream()):
+            r2, s2 = viterbi_tiles(tiles, lut, bits)
+            torch.cuda.synchronize()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert torch.equal(states, s2) and torch.equal(recon, r2)
