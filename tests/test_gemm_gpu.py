@@ -124,6 +124,30 @@ def test_bf16_gram_with_fewer_tiles_than_units(n, k):
     assert torch.equal(H, again)
 
 
+@pytest.mark.parametrize("dtype", (torch.float32, torch.bfloat16))
+def test_gram_without_room_for_its_partials_runs_whole(dtype):
+    n, k = 16384, 2048
+    print(f"[gemm] {dtype} gram n{n} k{k}, memory for the operands only", file=sys.stderr, flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(n + k)
+    X = torch.randn(n, k, device="cuda", generator=gen).to(dtype)
+    H, whole = torch.zeros(2, k, k, device="cuda")
+    lib, code = _native.lib(), int(dtype == torch.bfloat16)
+    nbytes = lib.qsrt_gemm_tn_workspace_bytes(H.data_ptr(), X.data_ptr(), X.data_ptr(), k, k, n, k, k, k, code)
+    assert nbytes > 32 << 20
+    _native.check(lib.qsrt_gemm_tn(whole.data_ptr(), X.data_ptr(), X.data_ptr(), None, k, k, n, k, k, k, 1.0 / n, code,
+                                   _native.stream_handle(X.device)), "qsrt_gemm_tn")
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (1 << 20)) / total)  # the allocator's own
+    try:
+        gemm.gram_(H, X, alpha=1.0 / n)
+        torch.cuda.synchronize()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert torch.equal(H, whole)
+
+
 def test_bf16_gram_full_size_matches_float64():
     """The Hessian capture at the config-4 shape: 16,384 bf16 rows x 7168
     channels.  Reference: the float64 product on the device (rocBLAS DGEMM),
