@@ -80,48 +80,65 @@ def test_bf16_gram_matches_float64(n, k):
 @pytest.mark.parametrize("n,k", [(5, 128), (64, 129), (1000, 4), (1000, 383), (8192, 256), (4096, 644), (16384, 130)])
 def test_f32_gram_matches_float64(n, k):
     """FP32 Gram: tiles on and above the diagonal and their mirror, whole or
-    in K ranges (the tall ones), at tile edges, into a non-zero H; the same
-    from call to call, and without a workspace equal to FP32 rounding."""
+    in K ranges (the tall ones), at tile edges, into a non-zero H whose rows
+    are padded to whole float4s (the ragged channel counts take the same
+    kernel, and leave the padding alone); the same from call to call, and
+    without a workspace equal to FP32 rounding."""
 
     print(f"[gemm] f32 gram n{n} k{k}", file=sys.stderr, flush=True)
     gen = torch.Generator(device="cuda").manual_seed(n + k)
-    X = torch.randn(n, k, device="cuda", generator=gen)
-    H0 = torch.randn(k, k, device="cuda", generator=gen)
-    want = H0.double() + X.double().T @ X.double() / n
+    ld = -(-k // 4) * 4 + 4
+    X = torch.randn(n, ld, device="cuda", generator=gen)[:, :k]
+    H0 = torch.randn(k, ld, device="cuda", generator=gen)
+    want = H0[:, :k].double() + X.double().T @ X.double() / n
+    lib = _native.lib()
+    nbytes = lib.qsrt_gemm_tn_workspace_bytes(H0.data_ptr(), X.data_ptr(), X.data_ptr(), k, k, n, ld, ld, ld, 0)
+    assert nbytes > 0 or n < 128  # K ranges of 64 rows at the least; a product that is no Gram asks for nothing
     # relative to the largest entry, as everywhere here: sums of n products of standard normals, each rounding 2^-24
     tol = max(1e-6, 2.0**-24 * n**0.5)
     H = H0.clone()
-    gemm.gram_(H, X, alpha=1.0 / n)
-    assert (H.double() - want).abs().max().item() <= tol * want.abs().max().item()
+    gemm.gram_(H[:, :k], X, alpha=1.0 / n)
+    assert (H[:, :k].double() - want).abs().max().item() <= tol * want.abs().max().item()
+    assert torch.equal(H[:, k:], H0[:, k:])
     again = H0.clone()
-    gemm.gram_(again, X, alpha=1.0 / n)
+    gemm.gram_(again[:, :k], X, alpha=1.0 / n)
     assert torch.equal(H, again)
-    if k % 4 == 0:  # the leading dimensions the C entry takes as they are
-        whole = H0.clone()
-        _native.check(_native.lib().qsrt_gemm_tn(whole.data_ptr(), X.data_ptr(), X.data_ptr(), None, k, k, n, k, k, k,
-                                                 1.0 / n, 0, _native.stream_handle(X.device)), "qsrt_gemm_tn")
-        assert (whole - H).abs().max().item() <= 2 * tol * want.abs().max().item()
+    whole = H0.clone()
+    _native.check(lib.qsrt_gemm_tn(whole.data_ptr(), X.data_ptr(), X.data_ptr(), None, k, k, n, ld, ld, ld, 1.0 / n, 0,
+                                   _native.stream_handle(X.device)), "qsrt_gemm_tn")
+    assert (whole - H).abs().max().item() <= 2 * tol * want.abs().max().item()
+    assert torch.equal(whole[:, k:], H0[:, k:])
 
 
 @pytest.mark.parametrize("n,k", [(130, 7), (129, 300), (8192, 256), (8191, 40), (4096, 1030), (300, 4200), (16384, 2056)])
 def test_bf16_gram_with_fewer_tiles_than_units(n, k):
     """Tile counts below the compute units': K ranges of every tile (or whole
-    tiles, at few rows), ragged rows and channels, into a non-zero H; equal
-    to the whole tiles to FP32 rounding and the same from call to call."""
+    tiles, where that is faster), ragged rows and channels, into a non-zero H with
+    padded rows; equal to the whole tiles to FP32 rounding and the same from
+    call to call."""
 
     print(f"[gemm] bf16 small gram n{n} k{k}", file=sys.stderr, flush=True)
     gen = torch.Generator(device="cuda").manual_seed(3 * n + k)
-    X = torch.randn(n, k, device="cuda", generator=gen).bfloat16()
-    H0 = torch.randn(k, k, device="cuda", generator=gen)
-    H0 = H0 + H0.T
-    want = H0.double() + X.double().T @ X.double() / n
+    ld = -(-k // 8) * 8 + 8
+    X = torch.randn(n, ld, device="cuda", generator=gen).bfloat16()[:, :k]
+    H0 = torch.randn(k, ld, device="cuda", generator=gen)
+    H0[:, :k] = H0[:, :k] + H0[:, :k].T.clone()
+    want = H0[:, :k].double() + X.double().T @ X.double() / n
+    lib = _native.lib()
+    nbytes = lib.qsrt_gemm_tn_workspace_bytes(H0.data_ptr(), X.data_ptr(), X.data_ptr(), k, k, n, ld, ld, ld, 1)
+    assert (nbytes > 0) == (k != 4200)  # 153 tiles of 5 stages stay whole, the others are split
     tol = max(1e-6, 2.0**-24 * n**0.5)  # FP32 sums of n exact products, relative to the largest entry
     H = H0.clone()
-    gemm.gram_(H, X, alpha=1.0 / n)
-    assert (H.double() - want).abs().max().item() <= tol * want.abs().max().item()
+    gemm.gram_(H[:, :k], X, alpha=1.0 / n)
+    assert (H[:, :k].double() - want).abs().max().item() <= tol * want.abs().max().item()
+    assert torch.equal(H[:, k:], H0[:, k:])
     again = H0.clone()
-    gemm.gram_(again, X, alpha=1.0 / n)
+    gemm.gram_(again[:, :k], X, alpha=1.0 / n)
     assert torch.equal(H, again)
+    whole = H0.clone()
+    _bf16_call(whole[:, :k], X, X, 1.0 / n)
+    assert torch.equal(whole, H) == (nbytes == 0)
+    assert (whole - H).abs().max().item() <= 2 * tol * want.abs().max().item()
 
 
 @pytest.mark.parametrize("dtype", (torch.float32, torch.bfloat16))

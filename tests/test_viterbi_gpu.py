@@ -137,13 +137,16 @@ def test_saturated_cost_paths_stay_closed(bits):
 @pytest.mark.parametrize("bits", (1, 2, 3, 4, 5, 6))
 def test_nan_tile_stays_a_path_and_leaves_its_neighbours(bits):
     """No path cost of a NaN tile compares; the boundary state is still a
-    state, and the other tiles of the launch are what they are without it."""
+    state and the tile's codewords a closed path, and the other tiles of the
+    launch are what they are without it."""
 
     _say(f"[viterbi] K{bits}: a NaN tile among 5")
     tiles = np.random.default_rng(900 + bits).standard_normal((5, 256)).astype(np.float32)
     want_recon, want = _gpu(tiles, bits, 128, 0 if bits == 2 else 1)
     tiles[2, 7] = np.nan
     recon, states = _gpu(tiles, bits, 128, 0 if bits == 2 else 1)
+    path = torch.from_numpy(states[2:3].astype(np.int64)) & 0xFFFF
+    assert torch.equal(reconstruct_trellis_states(path & ((1 << bits) - 1), bits).long() & 0xFFFF, path)
     others = [0, 1, 3, 4]
     assert np.array_equal(states[others], want[others])
     assert np.array_equal(recon[others], want_recon[others])
