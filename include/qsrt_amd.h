@@ -264,8 +264,8 @@ int qsrt_gemm_tn(float *C, const void *A, const void *B, const void *B2, int64_t
 
 /*
  * Device bytes qsrt_gemm_tn_ws wants as workspace for these arguments (0 when
- * the call has nothing to split: an f32 product that is not A^T A, or a tile
- * count that fills the device's compute units).
+ * the call splits nothing: an f32 product that is not A^T A, a tile count that
+ * fills the device's compute units, or few rows, where whole tiles are faster).
  */
 size_t qsrt_gemm_tn_workspace_bytes(const float *C, const void *A, const void *B, int64_t M, int64_t N, int64_t K,
                                     int64_t lda, int64_t ldb, int64_t ldc, int dtype);
@@ -276,11 +276,14 @@ size_t qsrt_gemm_tn_workspace_bytes(const float *C, const void *A, const void *B
  * the last round are split along K where that is faster and their partial
  * products, written to the workspace, are added to C in K order by a second
  * kernel on the same stream (the result is deterministic; it differs from the
- * unsplit sum only by FP32 rounding), or, at few rows, every tile sums its
- * rows in groups of 64 and needs no workspace.  f32 with A == B and no B2 (a Gram):
- * likewise for its 128 x 128 tiles on and above the diagonal, the only ones
- * computed.  A NULL or short workspace runs every tile whole, as
- * qsrt_gemm_tn does.  Same operator and call sites as qsrt_gemm_tn.
+ * unsplit sum only by FP32 rounding); with a NULL or short workspace those
+ * tiles run whole, as in qsrt_gemm_tn.  At few rows behind a whole round every
+ * tile instead sums its rows in groups of 64: qsrt_gemm_tn_workspace_bytes is 0
+ * then, whatever workspace is passed is left alone, and the result differs from
+ * qsrt_gemm_tn's by FP32 rounding.  f32 with A == B and no B2 (a Gram): only the
+ * 128 x 128 tiles on and above the diagonal are computed, split along K likewise;
+ * a NULL or short workspace runs them whole, as qsrt_gemm_tn does.  Same
+ * operator and call sites as qsrt_gemm_tn.
  */
 int qsrt_gemm_tn_ws(float *C, const void *A, const void *B, const void *B2, int64_t M, int64_t N, int64_t K,
                     int64_t lda, int64_t ldb, int64_t ldc, float alpha, int dtype, void *workspace,

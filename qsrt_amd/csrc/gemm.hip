@@ -599,7 +599,7 @@ int64_t bf16_tiles(bool sym, int64_t M, int64_t N) {
 // accumulators go to a workspace, and gram_f32_fixup adds them to C in K
 // order (deterministic).  MFMA-bound: 16384 x 2048 in all 256 tiles and one
 // workgroup per CU took 1.47 ms (0.59 of the FP32 matrix peak, half of it
-// redundant), this way 0.67 ms (0.69 of the peak, 6% redundant).
+// redundant), this way 0.64 ms (0.72 of the peak, 6% redundant).
 constexpr int64_t kGramPartial = 16 * kThreads;  // f32x4 per partial tile (64 KiB)
 
 // Sum of a tile's accumulators (16-row block i of every wave's 64 x 64 block) into C and, off the diagonal, into the
@@ -716,7 +716,14 @@ __global__ __launch_bounds__(kThreads) void gram_f32_fixup(float* __restrict__ C
 
 // K ranges per tile.  In units of one whole tile on a CU of its own at full MFMA rate: the CU with most ranges has n of
 // them, works at 0.6, 0.8 or 0.85 of that rate with one, two or three workgroups resident, and writes and reads back
-// n partials (128 KiB at a CU's share of HBM, 139 rows' worth of MFMA time).
+// n partials (128 KiB at a CU's share of HBM, 139 rows' worth of MFMA time).  Whole square tiles -> this, in us:
+//   rows     256 channels     1024            2048            7168
+//     64     17.6 -> 12.9     18.5 -> 13.7    20.6 -> 16.0    132 -> 89
+//    171     27.3 -> 15.7     28.5 -> 17.9    30.1 -> 25.4    217 -> 130
+//   1024     102 -> 18.9      109 -> 30.8     110 -> 73       939 -> 521
+//  16384     1454 -> 105      1468 -> 203     1462 -> 652     14,075 -> 6882
+// and at no size of 1 to 16384 rows by 256 to 7168 channels slower, nor without a workspace (2048 channels: 16.8 ->
+// 12.3 at one row, 1515 -> 1428 at 16384).
 int gram_f32_parts(int64_t tiles, int64_t K, int cus) {
     if (cus <= 0) return 1;
     double best = 0.0;
