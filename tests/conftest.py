@@ -2,6 +2,7 @@
 
 from __future__ import annotations
 
+import contextlib
 import sys
 from pathlib import Path
 
@@ -25,3 +26,30 @@ def pytest_collection_modifyitems(config, items):
     for item in items:
         if "gpu" in item.keywords:
             item.add_marker(skip)
+
+
+@contextlib.contextmanager
+def device_memory_left(nbytes: int):
+    """Torch's allocator has ``nbytes`` of device memory to give and no more
+    (its own limit, whatever the card still has; blocks under 1 MiB apart)."""
+
+    import torch
+
+    total = torch.cuda.get_device_properties(0).total_memory
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    taken = []
+    try:
+        torch.cuda.set_per_process_memory_fraction(torch.cuda.memory_reserved() / total)
+        size = 1 << 30
+        while size >= 1 << 20:  # what segments still in use have free
+            try:
+                taken.append(torch.empty(size, dtype=torch.uint8, device="cuda"))
+            except torch.OutOfMemoryError:
+                size //= 2
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + nbytes) / total)
+        yield
+        torch.cuda.synchronize()
+    finally:
+        del taken
+        torch.cuda.set_per_process_memory_fraction(1.0)

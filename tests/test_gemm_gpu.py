@@ -10,6 +10,7 @@ import numpy as np
 import pytest
 import torch
 
+from conftest import device_memory_left
 from qsrt_amd import _native, gemm
 
 pytestmark = pytest.mark.gpu
@@ -153,15 +154,8 @@ def test_gram_without_room_for_its_partials_runs_whole(dtype):
     assert nbytes > 32 << 20
     _native.check(lib.qsrt_gemm_tn(whole.data_ptr(), X.data_ptr(), X.data_ptr(), None, k, k, n, k, k, k, 1.0 / n, code,
                                    _native.stream_handle(X.device)), "qsrt_gemm_tn")
-    torch.cuda.synchronize()
-    torch.cuda.empty_cache()
-    total = torch.cuda.get_device_properties(0).total_memory
-    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (1 << 20)) / total)  # the allocator's own
-    try:
+    with device_memory_left(1 << 20):
         gemm.gram_(H, X, alpha=1.0 / n)
-        torch.cuda.synchronize()
-    finally:
-        torch.cuda.set_per_process_memory_fraction(1.0)
     assert torch.equal(H, whole)
 
 

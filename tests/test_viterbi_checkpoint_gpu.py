@@ -11,6 +11,7 @@ import numpy as np
 import pytest
 import torch
 
+from conftest import device_memory_left
 from oracle import tables as otables
 from oracle import viterbi as ov
 from qsrt_amd import _native
@@ -98,15 +99,9 @@ def test_checkpoints_that_do_not_fit_give_way_to_recorded_decisions(bits):
     recon, states = viterbi_tiles(tiles, lut, bits)
     recorded = torch.cuda.get_device_properties(0).multi_processor_count * (1 << 20 if bits == 4 else 2 << 20)
     assert recorded < _native.lib().qsrt_viterbi_workspace_bytes(bits, n)
-    torch.cuda.synchronize()
-    torch.cuda.empty_cache()
-    # the allocator's own limit, far below the card's memory; 64 MiB for the results and whole segments
-    limit = torch.cuda.memory_reserved() + recorded + (64 << 20)
-    torch.cuda.set_per_process_memory_fraction(limit / torch.cuda.get_device_properties(0).total_memory)
-    try:
-        with torch.cuda.stream(torch.cuda.Stream()):
-            r2, s2 = viterbi_tiles(tiles, lut, bits)
-            torch.cuda.synchronize()
-    finally:
-        torch.cuda.set_per_process_memory_fraction(1.0)
+    with device_memory_left(recorded + (64 << 20)), torch.cuda.stream(torch.cuda.Stream()):  # 64 MiB for the results
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        r2, s2 = viterbi_tiles(tiles, lut, bits)
+        assert torch.cuda.max_memory_allocated() - before < recorded + (64 << 20)
     assert torch.equal(states, s2) and torch.equal(recon, r2)
