@@ -105,3 +105,28 @@ def test_checkpoints_that_do_not_fit_give_way_to_recorded_decisions(bits):
         r2, s2 = viterbi_tiles(tiles, lut, bits)
         assert torch.cuda.max_memory_allocated() - before < recorded + (64 << 20)
     assert torch.equal(states, s2) and torch.equal(recon, r2)
+
+
+@pytest.mark.parametrize("bits", (2, 4))
+def test_captured_launch_keeps_its_workspace(bits):
+    """Replays with launches of the program's own in between, wider and narrower ones: each equals the eager result."""
+
+    n = 40
+    print(f"[viterbi] K{bits}: {n} tiles in a graph", file=sys.stderr, flush=True)
+    tiles = torch.randn((n, 256), device="cuda")
+    lut = sqg_xor_cheb_t12_bytes(bits).cuda()
+    want, want_states = viterbi_tiles(tiles, lut, bits)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        recon, states = viterbi_tiles(tiles, lut, bits)
+    for other in (300, 1, 600):
+        recon.zero_()
+        states.zero_()
+        side = torch.randn((other, 256), device="cuda")
+        first = viterbi_tiles(side, lut, bits)
+        graph.replay()
+        again = viterbi_tiles(side, lut, bits)
+        torch.cuda.synchronize()
+        assert torch.equal(states, want_states) and torch.equal(recon, want)
+        assert torch.equal(first[1], again[1])
